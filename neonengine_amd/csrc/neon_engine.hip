@@ -724,7 +724,8 @@ static void enqueue_rows(neon_ctx* ctx, int B, const int32_t* pos, const int32_t
     // batch >= 2: the top-k runs once per row before the experts, which then
     // group the rows by expert (each used expert's weights read once);
     // batch 1: the expert kernels choose from the logits themselves
-    const bool grouped = B >= 2 && B * c.top_k <= 64;
+    const bool grouped =
+        B >= 2 && (B * c.top_k <= 64 || xm_moe_wanted(B, c.top_k, c.n_experts));
     RouterArgs r;
     r.x = ctx->h; r.norm_w = w.mlp_norm; r.eps = c.rms_eps; r.xn_out = ctx->xn;
     r.W = w.router_w; r.bias = w.router_b; r.lg_out = ctx->router_lg;
@@ -751,7 +752,8 @@ static void enqueue_rows(neon_ctx* ctx, int B, const int32_t* pos, const int32_t
     m.residual = ctx->h; m.out = ctx->h; m.B = B; m.H = H; m.I = c.intermediate;
     m.k = c.top_k; m.alpha = c.swiglu_alpha; m.limit = c.swiglu_limit; m.err = ctx->dev_err;
     m.sync = sync;
-    if (grouped && moe_batched_supported(m)) launch_moe_batched(m, st);
+    if (grouped && xm_moe_supported(m)) launch_xm_moe(m, st);
+    else if (grouped && moe_batched_supported(m)) launch_moe_batched(m, st);
     else launch_moe(m, st);
   }
 }
@@ -1704,6 +1706,27 @@ static MoeLayerWs moe_layer_ws(int B, int E, int I, int k) {
   return w;
 }
 
+// Router and experts of one layer.  With several rows per expert: the
+// top-k of every row first (into the caller's idx / score, or ids_tmp: 8 bytes
+// per pair), so that rows that chose the same expert share one read of it;
+// else the expert kernels rank the logits themselves.  Same bits either way.
+static void launch_router_moe(RouterArgs& r, MoeArgs& m, int32_t* ids_tmp, hipStream_t st) {
+  MoeArgs g = m;
+  g.idx = r.idx = m.idx_out ? m.idx_out : ids_tmp;
+  g.score = r.score = m.score_out ? m.score_out : (float*)(ids_tmp + (size_t)m.B * m.k);
+  g.router_lg = nullptr;
+  static_assert(kXmMaxPairs * 8 <= kMoeSyncInts * 4, "the ids fit in the counters' place");
+  if (xm_moe_supported(g)) {
+    r.zero = nullptr; r.zero_n = 0;  // no arrival counters: their place may hold the ids
+    launch_router(r, st);
+    launch_xm_moe(g, st);
+    return;
+  }
+  r.idx = nullptr; r.score = nullptr;
+  launch_router(r, st);
+  launch_moe(m, st);
+}
+
 extern "C" size_t neon_moe_layer_workspace(int B, int E, int I, int k) {
   if (B < 1 || E < 1 || I < 1 || k < 1) return 0;
   return moe_layer_ws(B, E, I, k).total;
@@ -1735,7 +1758,6 @@ extern "C" neon_status neon_moe_layer(
   r.x = x; r.W = router_w; r.bias = router_b; r.lg_out = lg;
   r.B = B; r.E = E; r.H = H; r.k = k;
   r.zero = sync; r.zero_n = kMoeSyncZero;
-  launch_router(r, st);
   MoeArgs m;
   m.gu_codes = gu_codes; m.gu_scales = gu_scales; m.gu_bias = gu_bias;
   m.dn_codes = dn_codes; m.dn_scales = dn_scales; m.dn_bias = dn_bias;
@@ -1744,7 +1766,7 @@ extern "C" neon_status neon_moe_layer(
   m.out = out; m.B = B; m.H = H; m.I = I; m.k = k; m.alpha = alpha; m.limit = limit;
   m.err = device_status_word();
   m.sync = getenv("NEON_MOE_FUSED") && getenv("NEON_MOE_FUSED")[0] == '1' ? sync : nullptr;
-  launch_moe(m, st);
+  launch_router_moe(r, m, sync, st);
   KLAUNCHED();
 }
 
@@ -1754,7 +1776,7 @@ extern "C" neon_status neon_moe_layer(
 // to a kernel (on the host it is only a stand-in symbol): it resolves the
 // device address once per device with hipGetSymbolAddress and uses that.
 constexpr size_t kNoAllocScratchBytes = (size_t)4 << 20;  // 4 MiB
-static __device__ __align__(256) char scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) char scratch[kNoAllocScratchBytes + kXmMaxPairs * 8];  // + ids
 
 static std::mutex g_scratch_mu;
 static char* g_scratch_ptr[256];
@@ -1807,7 +1829,6 @@ extern "C" neon_status neon_moe_layer_noalloc(
   RouterArgs r;
   r.x = x; r.W = router_w; r.bias = router_b; r.lg_out = lg;
   r.B = B; r.E = E; r.H = H; r.k = k;
-  launch_router(r, st);
   MoeArgs m;
   m.gu_codes = gu_codes; m.gu_scales = gu_scales; m.gu_bias = gu_bias;
   m.dn_codes = dn_codes; m.dn_scales = dn_scales; m.dn_bias = dn_bias;
@@ -1815,7 +1836,7 @@ extern "C" neon_status neon_moe_layer_noalloc(
   m.score_out = score; m.E = E; m.xn = x; m.act = act; m.residual = residual;
   m.out = out; m.B = B; m.H = H; m.I = I; m.k = k; m.alpha = alpha; m.limit = limit;
   m.err = nullptr;  // the ids come from the in-kernel top-k: always in [0, E)
-  launch_moe(m, st);
+  launch_router_moe(r, m, (int32_t*)(base + kNoAllocScratchBytes), st);
   KLAUNCHED();
 }
 
@@ -1840,7 +1861,8 @@ extern "C" neon_status neon_moe_experts(
   m.score_out = nullptr; m.E = E; m.xn = x; m.act = act; m.residual = residual;
   m.out = out; m.B = B; m.H = H; m.I = I; m.k = k; m.alpha = alpha; m.limit = limit;
   m.err = device_status_word();
-  if (moe_batched_supported(m)) launch_moe_batched(m, S(stream));
+  if (xm_moe_supported(m)) launch_xm_moe(m, S(stream));
+  else if (moe_batched_supported(m)) launch_moe_batched(m, S(stream));
   else launch_moe(m, S(stream));
   KLAUNCHED();
 }

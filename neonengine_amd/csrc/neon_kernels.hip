@@ -17,19 +17,6 @@
 
 namespace neon {
 
-// Weight words are read once per step: a non-temporal load (streaming hint,
-// no reuse expected in the caches) measured 4.5% faster over the whole step
-// than a plain load.
-typedef uint32_t nt_u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint4 load_weight16(const void* p) {
-  const nt_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const nt_u32x4*>(p));
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint8_t load_weight1(const uint8_t* p) {
-  return __builtin_nontemporal_load(p);
-}
-
-
 // ===========================================================================
 // Deterministic init (identical integer/fp32 steps to the CPU oracle)
 // ===========================================================================
@@ -1701,11 +1688,6 @@ void launch_rope_apply(uint16_t* x, const int32_t* pos, const float* cos_t,
 constexpr int kMaxExperts = 256;
 constexpr int kMaxTopK = 16;
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 
 __device__ __forceinline__ float readlane_f(float v, int l) {
@@ -2505,7 +2487,8 @@ __global__ __launch_bounds__(1024) void k_moe_down(
 }
 
 // ===========================================================================
-// Batched experts (2 <= B, B k <= 64): rows that chose the same expert share
+// Batched experts (2 <= B, B k <= 64; few pairs per expert, see
+// xm_moe_supported for the others): rows that chose the same expert share
 // one read of its weights.  idx / score [B][k] come from the top-k kernel.
 // Pair q = b k + s is row b's slot s; lane q of a wave holds idx[q], and
 // __ballot(idx == e) lists the pairs of expert e in row order.
