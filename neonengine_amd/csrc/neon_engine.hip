@@ -110,6 +110,16 @@ struct neon_ctx {
   float *pf_lg = nullptr, *pf_score = nullptr, *pf_ybuf = nullptr;
   int32_t *pf_idx = nullptr, *pf_ltok = nullptr, *pf_lslot = nullptr, *pf_eoff = nullptr,
           *pf_tile_e = nullptr, *pf_tile_r0 = nullptr, *pf_ntiles = nullptr;
+  // exact prompt passes of many rows (enqueue_rows_many): scratch made by the
+  // first such pass
+  char* xg = nullptr;
+  int xg_rows = 0, xg_sub = 0;  // rows per pass, rows per attention launch
+  bool xg_failed = false;       // no memory for it: passes of kPromptRows rows
+  uint16_t *xg_h = nullptr, *xg_xn = nullptr, *xg_qkv = nullptr, *xg_q = nullptr, *xg_ao = nullptr;
+  float *xg_lg = nullptr, *xg_score = nullptr, *xg_po = nullptr, *xg_pml = nullptr;
+  int32_t *xg_idx = nullptr, *xg_pos = nullptr, *xg_seq = nullptr, *xg_arrive = nullptr;
+  void *xg_wp = nullptr, *xg_xp = nullptr;
+  XgMoeScratch xg_moe{};
   // next-token choice (temperature 0: greedy argmax)
   float temperature = 0.0f, top_p = 1.0f;
   uint64_t sample_seed = 0;
@@ -329,6 +339,7 @@ extern "C" void neon_ctx_destroy(neon_ctx* ctx) {
   if (ctx->vc) (void)hipFree(ctx->vc);
   if (ctx->work) (void)hipFree(ctx->work);
   if (ctx->pf) (void)hipFree(ctx->pf);
+  if (ctx->xg) (void)hipFree(ctx->xg);
   if (ctx->mx_w) (void)hipFree(ctx->mx_w);
   if (ctx->mx8_q) (void)hipFree(ctx->mx8_q);
   delete ctx;
@@ -501,6 +512,7 @@ static neon_status ctx_alloc(neon_ctx* ctx) {
   HIPCHK(ctx, hipDeviceSynchronize());
   HIPCHK(ctx, hipStreamCreateWithFlags(&ctx->cap_stream, hipStreamNonBlocking));
   HIPCHK(ctx, gemv_batched_prepare());
+  HIPCHK(ctx, xg_prepare());
   return NEON_OK;
 }
 
@@ -1101,6 +1113,146 @@ extern "C" neon_status neon_set_prefill_mode(neon_ctx* ctx, int mode) {
   return NEON_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Exact prompt passes of many rows: the same rows as enqueue_rows, each layer's
+// products over all of the pass's rows at once (neon_exact_prompt.hip), RoPE,
+// the KV append and attention over xg_sub of them at a time.  Bit-identical to
+// passes of kPromptRows rows.
+// ---------------------------------------------------------------------------
+// Rows of the largest pass (a longer one fills the 16-pair expert tiles better:
+// 512 rows x 4 experts / 32 = 64 pairs each) and from which a pass runs this
+// way: fewer rows than that take the decode kernels' 16 at a time.
+constexpr int kXgRows = 512, kXgMinRows = 24;
+
+static bool ensure_xg(neon_ctx* ctx) {
+  if (ctx->xg) return true;
+  if (ctx->xg_failed) return false;
+  const neon_config& c = ctx->cfg;
+  const size_t H = c.hidden, I = c.intermediate, E = c.n_experts, k = c.top_k;
+  const size_t qd = (size_t)c.n_heads * c.head_dim, qr = qd + 2 * (size_t)c.n_kv_heads * c.head_dim;
+  const int rows = std::min(kXgRows, kXgMaxPairs / c.top_k) / 16 * 16;
+  ctx->xg_failed = true;
+  if (!xg_supported(c.hidden, c.intermediate, (int)qd, (int)qr, c.n_experts) || rows < kXgMinRows)
+    return false;
+  // a ring cache takes the rows of one attention launch beside its window
+  int sub = std::min(128, rows);
+  for (int l = 0; l < c.n_layers; ++l)
+    if (ctx->kv_mask[l] >= 0) sub = std::min(sub, ctx->kv_rows[l] - c.sliding_window);
+  const size_t R = rows, pairs = R * k, S = std::max(ctx->s_full, ctx->s_slide);
+  size_t off = 0;
+  auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes); return o; };
+  const size_t o_h = take(R * H * 2), o_xn = take(R * H * 2), o_qkv = take(R * qr * 2),
+               o_q = take(R * qd * 2), o_ao = take(R * qd * 2), o_lg = take(R * E * 4),
+               o_sc = take(pairs * 4), o_idx = take(pairs * 4), o_pos = take(R * 4),
+               o_seq = take(R * 4), o_pair = take(pairs * 4), o_toff = take(257 * 4),
+               o_tile = take((size_t)xg_max_tiles((int)pairs, (int)E) * 4),
+               o_xt = take(xg_tile_bytes((int)pairs, (int)E, (int)H)),
+               o_yt = take(xg_tile_bytes((int)pairs, (int)E, (int)I)),
+               o_yb = take(pairs * H * 4),
+               o_wp = take(std::max(xg_packed_bytes((int)qr, (int)H), xg_packed_bytes((int)H, (int)qd))),
+               o_xp = take(std::max(xg_packed_bytes(rows, (int)H), xg_packed_bytes(rows, (int)qd))),
+               o_po = take((size_t)sub * c.n_heads * S * c.head_dim * 4),
+               o_pml = take((size_t)sub * c.n_heads * S * 2 * 4),
+               o_arr = take((size_t)sub * c.n_kv_heads * kAttnArriveStride * 4);
+  if (hipMalloc(&ctx->xg, off) != hipSuccess) {
+    ctx->xg = nullptr;
+    (void)hipGetLastError();  // handled: smaller passes need no scratch
+    return false;
+  }
+  char* P = ctx->xg;
+  if (hipMemset(P + o_arr, 0, off - o_arr) != hipSuccess) {
+    (void)hipFree(ctx->xg);
+    ctx->xg = nullptr;
+    return false;
+  }
+  ctx->xg_h = (uint16_t*)(P + o_h); ctx->xg_xn = (uint16_t*)(P + o_xn);
+  ctx->xg_qkv = (uint16_t*)(P + o_qkv); ctx->xg_q = (uint16_t*)(P + o_q);
+  ctx->xg_ao = (uint16_t*)(P + o_ao); ctx->xg_lg = (float*)(P + o_lg);
+  ctx->xg_score = (float*)(P + o_sc); ctx->xg_idx = (int32_t*)(P + o_idx);
+  ctx->xg_pos = (int32_t*)(P + o_pos); ctx->xg_seq = (int32_t*)(P + o_seq);
+  ctx->xg_moe.pair = (int32_t*)(P + o_pair); ctx->xg_moe.toff = (int32_t*)(P + o_toff);
+  ctx->xg_moe.tile = (uint32_t*)(P + o_tile); ctx->xg_moe.xt = P + o_xt;
+  ctx->xg_moe.yt = P + o_yt; ctx->xg_moe.ybuf = (float*)(P + o_yb);
+  ctx->xg_wp = P + o_wp; ctx->xg_xp = P + o_xp;
+  ctx->xg_po = (float*)(P + o_po); ctx->xg_pml = (float*)(P + o_pml);
+  ctx->xg_arrive = (int32_t*)(P + o_arr);
+  ctx->xg_rows = rows;
+  ctx->xg_sub = sub;
+  ctx->xg_failed = false;
+  return true;
+}
+
+static void enqueue_rows_many(neon_ctx* ctx, int R, hipStream_t st) {
+  const neon_config& c = ctx->cfg;
+  const int H = c.hidden, D = c.head_dim, qd = c.n_heads * D;
+  const int qr = qd + 2 * c.n_kv_heads * D;
+  launch_embed(ctx->tokens, ctx->tok_stride, ctx->xg_pos, ctx->xg_seq, ctx->embed, ctx->xg_h, H, R, st);
+  for (int l = 0; l < c.n_layers; ++l) {
+    const LayerW& w = ctx->layers[l];
+    const bool sliding = (l % 2 == 0) && c.sliding_window > 0;  // HFC:75-78
+    uint16_t* kc_l = ctx->kc + ctx->kv_off[l];
+    uint16_t* vc_l = ctx->vc + ctx->kv_off[l];
+    launch_rmsnorm(ctx->xg_h, w.attn_norm, ctx->xg_xn, R, H, c.rms_eps, st);
+    launch_xg_dense(w.wqkv, w.bqkv, ctx->xg_xn, ctx->xg_qkv, R, qr, H, false, ctx->xg_wp, ctx->xg_xp, st);
+    for (int r0 = 0; r0 < R; r0 += ctx->xg_sub) {
+      const int n = std::min(ctx->xg_sub, R - r0);
+      launch_mx_rope_append(ctx->xg_qkv + (size_t)r0 * qr, ctx->xg_pos + r0, ctx->xg_seq + r0,
+                            ctx->cos_t, ctx->sin_t, ctx->xg_q + (size_t)r0 * qd, kc_l, vc_l, n,
+                            c.n_heads, c.n_kv_heads, ctx->kv_rows[l], ctx->kv_mask[l], st);
+      AttnArgs a;
+      a.q = ctx->xg_q + (size_t)r0 * qd; a.kc = kc_l; a.vc = vc_l; a.sinks = w.sinks;
+      a.pos = ctx->xg_pos + r0; a.out = ctx->xg_ao + (size_t)r0 * qd; a.part_o = ctx->xg_po;
+      a.part_ml = ctx->xg_pml; a.seq = ctx->xg_seq + r0; a.arrive = ctx->xg_arrive;
+      a.B = n; a.Hq = c.n_heads; a.Hkv = c.n_kv_heads;
+      a.T_max = ctx->kv_rows[l]; a.key_mask = ctx->kv_mask[l];
+      a.window = sliding ? c.sliding_window : 0;
+      a.S = sliding ? ctx->s_slide : ctx->s_full; a.q_stride = qd;
+      launch_attn(a, st);
+    }
+    launch_xg_dense(w.wo, w.bo, ctx->xg_ao, ctx->xg_h, R, H, qd, true, ctx->xg_wp, ctx->xg_xp, st);
+    RouterArgs r;
+    r.x = ctx->xg_h; r.norm_w = w.mlp_norm; r.eps = c.rms_eps; r.xn_out = ctx->xg_xn;
+    r.W = w.router_w; r.bias = w.router_b; r.lg_out = ctx->xg_lg;
+    r.idx = ctx->xg_idx; r.score = ctx->xg_score;
+    r.B = R; r.E = c.n_experts; r.H = H; r.k = c.top_k;
+    launch_router(r, st);
+    MoeArgs m;
+    m.gu_codes = w.gu_codes; m.gu_scales = w.gu_scales; m.gu_bias = w.gu_bias;
+    m.dn_codes = w.dn_codes; m.dn_scales = w.dn_scales; m.dn_bias = w.dn_bias;
+    m.router_lg = nullptr; m.idx = ctx->xg_idx; m.score = ctx->xg_score;
+    m.idx_out = nullptr; m.score_out = nullptr; m.E = c.n_experts; m.xn = ctx->xg_xn;
+    m.act = nullptr; m.residual = ctx->xg_h; m.out = ctx->xg_h; m.B = R; m.H = H;
+    m.I = c.intermediate; m.k = c.top_k; m.alpha = c.swiglu_alpha; m.limit = c.swiglu_limit;
+    m.err = ctx->dev_err;
+    launch_xg_moe(m, ctx->xg_moe, st);
+  }
+}
+
+// Prompt rows (position rp[i] of sequence rs[i], each sequence's in order)
+// through every layer: `per` = 1 one at a time, else in passes of many rows,
+// or of kPromptRows where few are left.  rp / rs stay alive until the stream
+// is synchronised.
+static neon_status prompt_rows(neon_ctx* ctx, const int32_t* rp, const int32_t* rs, size_t n_rows,
+                               int per, hipStream_t st) {
+  for (size_t r0 = 0; r0 < n_rows;) {
+    const size_t left = n_rows - r0;
+    if (per > 1 && left >= (size_t)kXgMinRows && ensure_xg(ctx)) {
+      const int R = (int)std::min<size_t>(ctx->xg_rows, left);
+      HIPCHK(ctx, hipMemcpyAsync(ctx->xg_pos, rp + r0, R * 4, hipMemcpyHostToDevice, st));
+      HIPCHK(ctx, hipMemcpyAsync(ctx->xg_seq, rs + r0, R * 4, hipMemcpyHostToDevice, st));
+      enqueue_rows_many(ctx, R, st);
+      r0 += R;
+    } else {
+      const int R = (int)std::min<size_t>(per, left);
+      HIPCHK(ctx, hipMemcpyAsync(ctx->row_pos, rp + r0, R * 4, hipMemcpyHostToDevice, st));
+      HIPCHK(ctx, hipMemcpyAsync(ctx->row_seq, rs + r0, R * 4, hipMemcpyHostToDevice, st));
+      enqueue_rows(ctx, R, ctx->row_pos, ctx->row_seq, st);
+      r0 += R;
+    }
+  }
+  return NEON_OK;
+}
+
 // The prompt pass shared by neon_prefill and neon_prefill_ragged: sequence
 // b's prompt is ids[start[b] .. start[b] + lens[b]).  Each sequence keeps its
 // own position: rows 0 .. lens[b]-2 fill its KV cache, then one decode step
@@ -1160,23 +1312,17 @@ static neon_status prefill_seqs(neon_ctx* ctx, const int32_t* ids, const int32_t
       if (lens[b] > 1) enqueue_prefill_rows(ctx, b, lens[b] - 1, st);
   } else {
     // NEON_PREFILL_CHUNKED: the (position, sequence) rows of all sequences,
-    // each sequence's in position order, kPromptRows at a time through the
-    // batched decode kernels (their k / v fill the cache before the pass's
-    // attention, so row p attends to its sequence's keys <= p).
-    // NEON_PREFILL_STEPWISE with different lengths: the same rows one at a
-    // time.  The rows are staged up front and stay alive until the stream is
-    // synchronised below.
+    // each sequence's in position order, many at a time (their k / v fill the
+    // cache before their attention, so row p attends to its sequence's keys
+    // <= p).  NEON_PREFILL_STEPWISE with different lengths: the same rows one
+    // at a time.  The rows are staged up front and stay alive until the stream
+    // is synchronised below.
     const int per = ctx->prefill_mode == NEON_PREFILL_STEPWISE ? 1 : kPromptRows;
     std::vector<int32_t> rp, rs;
     for (int b = 0; b < batch; ++b)
       for (int p = 0; p + 1 < lens[b]; ++p) { rp.push_back(p); rs.push_back(b); }
-    const size_t n_rows = rp.size();
-    for (size_t r0 = 0; r0 < n_rows; r0 += per) {
-      const int R = (int)std::min<size_t>(per, n_rows - r0);
-      HIPCHK(ctx, hipMemcpyAsync(ctx->row_pos, &rp[r0], R * 4, hipMemcpyHostToDevice, st));
-      HIPCHK(ctx, hipMemcpyAsync(ctx->row_seq, &rs[r0], R * 4, hipMemcpyHostToDevice, st));
-      enqueue_rows(ctx, R, ctx->row_pos, ctx->row_seq, st);
-    }
+    neon_status ps = prompt_rows(ctx, rp.data(), rs.data(), rp.size(), per, st);
+    if (ps != NEON_OK) return ps;
     HIPCHK(ctx, hipStreamSynchronize(st));  // rp and rs die here
   }
   HIPCHK(ctx, hipGetLastError());
@@ -1463,12 +1609,8 @@ extern "C" neon_status neon_seq_add(neon_ctx* ctx, const int32_t* ids, int n, in
     const int per = ctx->prefill_mode == NEON_PREFILL_STEPWISE ? 1 : kPromptRows;
     std::vector<int32_t> rp, rs;
     for (int p = 0; p < n; ++p) { rp.push_back(p); rs.push_back(slot); }
-    for (int r0 = 0; r0 + 1 < n; r0 += per) {
-      const int R = std::min(per, n - 1 - r0);
-      HIPCHK(ctx, hipMemcpyAsync(ctx->row_pos, &rp[r0], R * 4, hipMemcpyHostToDevice, st));
-      HIPCHK(ctx, hipMemcpyAsync(ctx->row_seq, &rs[r0], R * 4, hipMemcpyHostToDevice, st));
-      enqueue_rows(ctx, R, ctx->row_pos, ctx->row_seq, st);
-    }
+    neon_status ps = prompt_rows(ctx, rp.data(), rs.data(), (size_t)n - 1, per, st);
+    if (ps != NEON_OK) return ps;
     HIPCHK(ctx, hipStreamSynchronize(st));  // rp and rs die here
   }
   // the last prompt token as a one-row step of this sequence alone: its

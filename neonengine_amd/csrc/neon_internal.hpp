@@ -275,6 +275,30 @@ bool xm_moe_wanted(int B, int k, int E);
 bool xm_moe_supported(const MoeArgs& a);
 void launch_xm_moe(const MoeArgs& a, hipStream_t st);
 
+// ---- exact prompt pass (neon_exact_prompt.hip): many rows at once, bit-identical
+// to one row at a time
+constexpr int kXgMaxPairs = 4096;  // (row, slot) pairs of one expert call
+struct XgMoeScratch {
+  int32_t *pair, *toff;  // [pairs], [257]
+  uint32_t* tile;        // [xg_max_tiles]
+  void *xt, *yt;         // input tiles of gate_up and of down (xg_tile_bytes)
+  float* ybuf;           // [pairs][H]
+};
+bool xg_supported(int H, int I, int qd, int qkv_rows, int E);
+hipError_t xg_prepare();
+size_t xg_packed_bytes(int rows, int K);
+int xg_max_tiles(int pairs, int E);
+size_t xg_tile_bytes(int pairs, int E, int K);
+// y = bf16(x W^T + bias), with resid y = bf16(y + bf16(x W^T + bias)); wp / xp
+// hold the packed operands (xg_packed_bytes of N and of M rows)
+void launch_xg_dense(const uint16_t* W, const uint16_t* bias, const uint16_t* x, uint16_t* y, int M,
+                     int N, int K, bool resid, void* wp, void* xp, hipStream_t st);
+// the experts of a.B rows (idx / score given) added into a.out, which is also the residual
+void launch_xg_moe(const MoeArgs& a, const XgMoeScratch& s, hipStream_t st);
+// h[t] = bf16(h[t] + bf16(sum_s score ybuf)) over the slots in order
+void launch_moe_combine(const float* ybuf, const float* score, const int32_t* idx, int M, int E,
+                        int k, int H, uint16_t* h, hipStream_t st);
+
 // ---- attention ------------------------------------------------------------------
 struct AttnArgs {
   const uint16_t* q;      // rotated q [B][q_stride] (head h at h*D)

@@ -1469,12 +1469,16 @@ void launch_moe_prefill(const MoePrefillArgs& a, hipStream_t st) {
   else
     hipLaunchKernelGGL((k_gemm<GEMM_SCATTER, true, true>), dim3((a.H + kGN - 1) / kGN, max_tiles),
                        dim3(256), 0, st, p);
-  if (a.H % 8 == 0 && a.k == 4)  // the gpt-oss top-4
-    hipLaunchKernelGGL(k_moe_combine8<4>, dim3(a.M), dim3(min(384, (a.H / 8 + 63) / 64 * 64)),
-                       0, st, a.ybuf, a.score, a.idx, a.E, a.H, a.h);
+  launch_moe_combine(a.ybuf, a.score, a.idx, a.M, a.E, a.k, a.H, a.h, st);
+}
+
+void launch_moe_combine(const float* ybuf, const float* score, const int32_t* idx, int M, int E,
+                        int k, int H, uint16_t* h, hipStream_t st) {
+  if (H % 8 == 0 && k == 4)  // the gpt-oss top-4
+    hipLaunchKernelGGL(k_moe_combine8<4>, dim3(M), dim3(min(384, (H / 8 + 63) / 64 * 64)), 0, st,
+                       ybuf, score, idx, E, H, h);
   else
-    hipLaunchKernelGGL(k_moe_combine, dim3(a.M), dim3(256), 0, st, a.ybuf, a.score, a.idx, a.E,
-                       a.k, a.H, a.h);
+    hipLaunchKernelGGL(k_moe_combine, dim3(M), dim3(256), 0, st, ybuf, score, idx, E, k, H, h);
 }
 
 int moe_prefill_max_tiles(int M, int k, int E) {

@@ -60,3 +60,38 @@ def test_experts_batch_bits(B, E, H, I, k, special):
             ne.device_check()
     same = (got.view(torch.int16) == ref.view(torch.int16)) | (got.isnan() & ref.isnan())
     assert bool(same.all()), int((~same).sum())
+
+
+SMALL = dict(n_layers=2, hidden=512, n_heads=16, n_kv_heads=2, head_dim=64, n_experts=8, top_k=4,
+             intermediate=512, vocab=1024, sliding_window=128, max_seq=768, max_batch=4)
+
+
+@pytest.mark.parametrize("lens,over", [
+    ([25], {}),                                    # the fewest rows of a wide pass
+    ([145], {}),                                   # a second attention launch of 16 rows
+    ([530], {}),                                   # a pass of 512 rows, then 17 by 16s; ring wraps
+    ([40, 3, 1, 90], {}),                          # several sequences in one pass
+    ([200], dict(sliding_window=40)),              # ring of 64 rows: 24 rows per attention launch
+    ([70], dict(hidden=192, intermediate=320)),    # 6 and 10 units: short rows, empty chains
+    ([70], dict(hidden=2112, intermediate=2176, n_experts=4)),  # 66 and 68 units: second passes
+    ([60], dict(n_experts=1, top_k=1, sliding_window=0)),       # one expert, every layer full
+])
+def test_prompt_passes_bits(lens, over):
+    """Prompt rows many at a time against every token as a step of its own:
+    the same logits after the prompt and after four more steps."""
+    torch_cuda()
+    print(f"prompt passes lens={lens} {over}", flush=True)
+    cfg = ne.config_preset("gpt-oss-20b", **dict(SMALL, **over))
+    prompts = [[(37 * i + 11 * b + 5) % 1024 for i in range(n)] for b, n in enumerate(lens)]
+    got = []
+    for mode in (ne.PREFILL_CHUNKED, ne.PREFILL_STEPWISE):
+        eng = ne.Engine(cfg)
+        eng.init_random(5)
+        eng.set_prefill_mode(mode)
+        eng.prefill(prompts)
+        first = eng.read_logits()
+        eng.decode(4)
+        got.append((first, eng.read_logits(), eng.read_tokens()))
+        eng.close()
+    for a, b in zip(*got):
+        assert a.tobytes() == b.tobytes()
