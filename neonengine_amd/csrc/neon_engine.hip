@@ -117,7 +117,7 @@ struct neon_ctx {
   bool xg_failed = false;       // no memory for it: passes of kPromptRows rows
   uint16_t *xg_h = nullptr, *xg_xn = nullptr, *xg_qkv = nullptr, *xg_q = nullptr, *xg_ao = nullptr;
   float *xg_lg = nullptr, *xg_score = nullptr, *xg_po = nullptr, *xg_pml = nullptr;
-  int32_t *xg_idx = nullptr, *xg_pos = nullptr, *xg_seq = nullptr, *xg_arrive = nullptr;
+  int32_t *xg_idx = nullptr, *xg_pos = nullptr, *xg_seq = nullptr;
   void *xg_wp = nullptr, *xg_xp = nullptr;
   XgMoeScratch xg_moe{};
   // next-token choice (temperature 0: greedy argmax)
@@ -1152,19 +1152,13 @@ static bool ensure_xg(neon_ctx* ctx) {
                o_wp = take(std::max(xg_packed_bytes((int)qr, (int)H), xg_packed_bytes((int)H, (int)qd))),
                o_xp = take(std::max(xg_packed_bytes(rows, (int)H), xg_packed_bytes(rows, (int)qd))),
                o_po = take((size_t)sub * c.n_heads * S * c.head_dim * 4),
-               o_pml = take((size_t)sub * c.n_heads * S * 2 * 4),
-               o_arr = take((size_t)sub * c.n_kv_heads * kAttnArriveStride * 4);
+               o_pml = take((size_t)sub * c.n_heads * S * 2 * 4);
   if (hipMalloc(&ctx->xg, off) != hipSuccess) {
     ctx->xg = nullptr;
     (void)hipGetLastError();  // handled: smaller passes need no scratch
     return false;
   }
   char* P = ctx->xg;
-  if (hipMemset(P + o_arr, 0, off - o_arr) != hipSuccess) {
-    (void)hipFree(ctx->xg);
-    ctx->xg = nullptr;
-    return false;
-  }
   ctx->xg_h = (uint16_t*)(P + o_h); ctx->xg_xn = (uint16_t*)(P + o_xn);
   ctx->xg_qkv = (uint16_t*)(P + o_qkv); ctx->xg_q = (uint16_t*)(P + o_q);
   ctx->xg_ao = (uint16_t*)(P + o_ao); ctx->xg_lg = (float*)(P + o_lg);
@@ -1175,14 +1169,14 @@ static bool ensure_xg(neon_ctx* ctx) {
   ctx->xg_moe.yt = P + o_yt; ctx->xg_moe.ybuf = (float*)(P + o_yb);
   ctx->xg_wp = P + o_wp; ctx->xg_xp = P + o_xp;
   ctx->xg_po = (float*)(P + o_po); ctx->xg_pml = (float*)(P + o_pml);
-  ctx->xg_arrive = (int32_t*)(P + o_arr);
   ctx->xg_rows = rows;
   ctx->xg_sub = sub;
   ctx->xg_failed = false;
   return true;
 }
 
-static void enqueue_rows_many(neon_ctx* ctx, int R, hipStream_t st) {
+// pos: the rows' positions on the host
+static void enqueue_rows_many(neon_ctx* ctx, const int32_t* pos, int R, hipStream_t st) {
   const neon_config& c = ctx->cfg;
   const int H = c.hidden, D = c.head_dim, qd = c.n_heads * D;
   const int qr = qd + 2 * c.n_kv_heads * D;
@@ -1202,12 +1196,12 @@ static void enqueue_rows_many(neon_ctx* ctx, int R, hipStream_t st) {
       AttnArgs a;
       a.q = ctx->xg_q + (size_t)r0 * qd; a.kc = kc_l; a.vc = vc_l; a.sinks = w.sinks;
       a.pos = ctx->xg_pos + r0; a.out = ctx->xg_ao + (size_t)r0 * qd; a.part_o = ctx->xg_po;
-      a.part_ml = ctx->xg_pml; a.seq = ctx->xg_seq + r0; a.arrive = ctx->xg_arrive;
+      a.part_ml = ctx->xg_pml; a.seq = ctx->xg_seq + r0;
       a.B = n; a.Hq = c.n_heads; a.Hkv = c.n_kv_heads;
       a.T_max = ctx->kv_rows[l]; a.key_mask = ctx->kv_mask[l];
       a.window = sliding ? c.sliding_window : 0;
       a.S = sliding ? ctx->s_slide : ctx->s_full; a.q_stride = qd;
-      launch_attn(a, st);
+      launch_xa_attn(a, *std::max_element(pos + r0, pos + r0 + n) + 1, st);
     }
     launch_xg_dense(w.wo, w.bo, ctx->xg_ao, ctx->xg_h, R, H, qd, true, ctx->xg_wp, ctx->xg_xp, st);
     RouterArgs r;
@@ -1240,7 +1234,7 @@ static neon_status prompt_rows(neon_ctx* ctx, const int32_t* rp, const int32_t* 
       const int R = (int)std::min<size_t>(ctx->xg_rows, left);
       HIPCHK(ctx, hipMemcpyAsync(ctx->xg_pos, rp + r0, R * 4, hipMemcpyHostToDevice, st));
       HIPCHK(ctx, hipMemcpyAsync(ctx->xg_seq, rs + r0, R * 4, hipMemcpyHostToDevice, st));
-      enqueue_rows_many(ctx, R, st);
+      enqueue_rows_many(ctx, rp + r0, R, st);
       r0 += R;
     } else {
       const int R = (int)std::min<size_t>(per, left);

@@ -334,6 +334,9 @@ constexpr int kAttnArriveStride = 64;
 // decode attention of the matrix-core steps (same partials and merge as launch_attn)
 void launch_mx_attn(const AttnArgs& a, hipStream_t st);
 void launch_attn_merge(const AttnArgs& a, hipStream_t st);
+// launch_attn on the fp32 matrix instructions (neon_exact_attn.hip), bit-
+// identical; max_keys bounds the keys of a row (its position + 1)
+void launch_xa_attn(const AttnArgs& a, int max_keys, hipStream_t st);
 void launch_attn(const AttnArgs& a, hipStream_t st);
 // number of key splits used for a cache of T_max rows (window 0 = full layer)
 int attn_splits(int T_max, int window);

@@ -95,3 +95,39 @@ def test_prompt_passes_bits(lens, over):
         eng.close()
     for a, b in zip(*got):
         assert a.tobytes() == b.tobytes()
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,window", [
+    (64, 8, 8, 130, 0),    # one query head per kv head, one split of up to 3 chunks
+    (72, 16, 8, 64, 0),    # two heads; one chunk
+    (33, 16, 4, 700, 0),   # four heads, 11 splits of one chunk, most of them empty early on
+    (5, 64, 8, 2200, 0),   # 32 splits of one or two chunks
+    (20, 64, 8, 300, 77),  # windows that start inside a chunk
+])
+def test_attention_batch_bits(B, Hq, Hkv, T, window):
+    """Batches large enough for the matrix form against one row at a time, with
+    positions at the ends of chunks and rows past them that hold NaN."""
+    torch = torch_cuda()
+    print(f"attention B={B} Hq={Hq} Hkv={Hkv} T={T} window={window}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(B + T)
+
+    def bf(*shape):
+        return torch.randn(shape, generator=g, device="cuda").to(torch.bfloat16)
+
+    q, k, v, sinks = bf(B, Hq * 64), bf(B, Hkv, T, 64), bf(B, Hkv, T, 64), bf(Hq)
+    ends = [0, 1, 62, 63, 64, 65, 127, 128, T - 1, T // 2]
+    pos = [min(ends[b % len(ends)] + 64 * (b // len(ends)), T - 1) for b in range(B)]
+    for b, p in enumerate(pos):
+        k[b, :, p + 1:], v[b, :, p + 1:] = float("nan"), float("nan")
+    v[1, 0, 0, 5], k[2, 0, 0, 7] = float("inf"), float("nan")
+    pt = torch.tensor(pos, dtype=torch.int32, device="cuda")
+
+    def run(lo, hi):
+        out = torch.empty((hi - lo, Hq * 64), dtype=torch.bfloat16, device="cuda")
+        ne.attn_decode(q[lo:hi], k[lo:hi], v[lo:hi], sinks, pt[lo:hi].contiguous(), out, hi - lo,
+                       Hq, Hkv, 64, T, window)
+        return out
+
+    got, ref = run(0, B), torch.cat([run(b, b + 1) for b in range(B)])
+    same = (got.view(torch.int16) == ref.view(torch.int16)) | (got.isnan() & ref.isnan())
+    assert bool(same.all()), int((~same).sum())
