@@ -131,3 +131,23 @@ def test_attention_batch_bits(B, Hq, Hkv, T, window):
     got, ref = run(0, B), torch.cat([run(b, b + 1) for b in range(B)])
     same = (got.view(torch.int16) == ref.view(torch.int16)) | (got.isnan() & ref.isnan())
     assert bool(same.all()), int((~same).sum())
+
+
+@pytest.mark.parametrize("V,T,p", [(1, 1.0, 0.9), (1000, 0.7, 0.9), (66560, 1.3, 0.999),
+                                   (70001, 0.5, 1.0), (201088, 0.8, 0.95)])
+def test_sampling_rows_alike(V, T, p):
+    """Rows of a batch draw what they draw alone, and equal logits (every value
+    at the threshold) stay in range."""
+    torch = torch_cuda()
+    print(f"sampling V={V} T={T} top_p={p}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(V)
+    lg = 3 * torch.randn((3, V), generator=g, device="cuda")
+    lg[2] = 0.25
+    pos = torch.tensor([5, 6, 7], dtype=torch.int32, device="cuda")
+    out, again = torch.empty_like(pos), torch.empty_like(pos)
+    ne.sample_logits(lg, 3, V, T, p, 11, pos, out)
+    ne.sample_logits(lg, 3, V, T, p, 11, pos, again)
+    assert out.tolist() == again.tolist() and all(0 <= i < V for i in out.tolist())
+    one = torch.empty(1, dtype=torch.int32, device="cuda")
+    ne.sample_logits(lg[:1].contiguous(), 1, V, T, p, 11, pos[:1].contiguous(), one)
+    assert one.item() == out[0].item()
