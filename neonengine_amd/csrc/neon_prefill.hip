@@ -17,6 +17,7 @@
 #include "neon_internal.hpp"
 
 #include <cstdlib>
+#include <type_traits>
 
 namespace neon {
 
@@ -53,16 +54,16 @@ void launch_embed_rows(const int32_t* ids, int M, const uint16_t* embed,
 // wave a 64 x 64 tile of 2 x 2 MFMA 32x32x16 blocks.  Both operands are
 // "row of the matrix, 8 consecutive k" per lane (lane l: row l % 32, k
 // 8 (l / 32) .. + 8), so A [M][K] and W [N][K] are staged the same way:
-// global -> registers (next step) -> LDS (double buffer, row stride 40 bf16
+// global -> registers (steps ahead) -> LDS (double buffer, row stride 72 bf16
 // so rows spread over the banks) -> ds_read_b128 operands.
 //
 // Rows past M or N read a clamped valid row and are never stored.  K must be
 // a multiple of 32; when it is not one of 64, the last step's upper 32
 // elements are zeros (a zero A value and a zero code add nothing).  With FP4,
 // W is an MXFP4 matrix (codes [N][K/2], scales [N][K/32]); a thread stages
-// one scale block (32 values) of one row per step, dequantised as
-// E2M1 (v_cvt_scalef32_pk_f32_fp4, exact) x 2^(s-127) (ldexp, exact) and
-// rounded to bf16 (exact: every such value is a bf16 value or overflows).
+// one scale block (32 values) of one row per step, dequantised to bf16 as
+// E2M1 x 2^(s-127) (fp4x16_to_bf16; exact: every such value is a bf16 value or
+// overflows).
 //
 // Grouped (MoE) form: blockIdx.y is a tile of the expert-sorted row list;
 // tile_e / tile_r0 give its expert and first list row, and rows past the
@@ -111,28 +112,24 @@ __device__ __forceinline__ float swiglu_clamp_p(float g, float u, float alpha, f
   return __fmul_rn(__fadd_rn(u, 1.0f), __fmul_rn(g, sig));
 }
 
-// 16 E2M1 values of 8 code bytes, times 2^(s - 127), as 16 bf16 (two uint4)
+// 16 E2M1 values of 8 code bytes, times 2^(s - 127), as 16 bf16 (two uint4).
+// v_cvt_scalef32_pk_bf16_fp4 reads the scale's exponent field alone, so s << 23
+// serves every s: its 256 scales x 256 code bytes are the exact products rounded
+// to bf16 (s = 0 and results below the normals included), and s = 255 gives NaN.
+// One instruction for two values in place of a conversion, two ldexp, the NaN
+// selects and a pack, which were ~200 vector instructions of a K step and the
+// bound of the FP4 tiles (32 experts, 333 rows, both GEMMs and the grouping:
+// 315 -> 281 us).
 __device__ __forceinline__ void fp4x16_to_bf16(u32x2_t c, uint32_t s, u32x4_t& lo, u32x4_t& hi) {
-  const int ex = (int)s - 127;
-  const bool nan = s == 0xFFu;
+  const float sc = __uint_as_float(s << 23);
   uint32_t o[8];
   const uint32_t w[2] = {c.x, c.y};
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      float2_v v;
-      switch (b) {
-        case 0: v = fp4x2_to_f32<0>(w[q]); break;
-        case 1: v = fp4x2_to_f32<1>(w[q]); break;
-        case 2: v = fp4x2_to_f32<2>(w[q]); break;
-        default: v = fp4x2_to_f32<3>(w[q]); break;
-      }
-      float a = __builtin_amdgcn_ldexpf(v.x, ex), bb = __builtin_amdgcn_ldexpf(v.y, ex);
-      a = nan ? __builtin_nanf("") : a;
-      bb = nan ? __builtin_nanf("") : bb;
-      o[q * 4 + b] = pack_bf2(a, bb);
-    }
+    o[q * 4 + 0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[q], sc, 0));
+    o[q * 4 + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[q], sc, 1));
+    o[q * 4 + 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[q], sc, 2));
+    o[q * 4 + 3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[q], sc, 3));
   }
   lo = u32x4_t{o[0], o[1], o[2], o[3]};
   hi = u32x4_t{o[4], o[5], o[6], o[7]};
@@ -242,10 +239,10 @@ __device__ __forceinline__ void gemm_epilogue(const f32x16_t (&acc)[2][2], const
 }
 
 template <int MODE, bool FP4, bool GROUPED>
-__global__ __launch_bounds__(256) void k_gemm(GemmParams p) {
+__global__ __launch_bounds__(256, 2) void k_gemm(GemmParams p) {
   __shared__ __align__(16) uint16_t As[2][kGM * kGS];
   __shared__ __align__(16) uint16_t Ws[2][kGN * kGS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int n0 = blockIdx.x * kGN;
   int e = 0, r0, rows;  // rows: valid A rows of this tile (from r0)
@@ -292,27 +289,34 @@ __global__ __launch_bounds__(256) void k_gemm(GemmParams p) {
       wrow[i] = p.W + (size_t)min(n0 + r, p.N - 1) * p.ldw + pc;
     }
   }
-  const u32x4_t z4 = {0u, 0u, 0u, 0u};
-  u32x4_t ra[4], rw[4] = {z4, z4, z4, z4};
-  u32x4_t rc = z4;
-  uint32_t rs = 127;
-  // the loads of the step at element ko; pieces past K are zeros
-  auto load_step = [&](int ko) {
-    const bool aok = ko + pc < K;
+  // Steps on their way: a step's loads are issued D steps before it is staged
+  // (one step ahead left each step waiting for a memory round trip; 32 experts of
+  // 33 / 333 / 2047 rows, both GEMMs and the grouping, 306 / 338 / 783 us with it
+  // and 235 / 315 / 751 us with four FP4 steps on their way).  All loads
+  // are unconditional, with addresses held inside the row: one under a
+  // condition makes the zeros of its other side wait for the loads in flight.
+  // Pieces past K (the upper half of the last step when K is odd in 32s)
+  // become zeros when they are staged.
+  constexpr int D = FP4 ? 4 : 2;  // even: the LDS buffer of a set is fixed
+  u32x4_t ra[D][4], rw[D][FP4 ? 1 : 4];
+  uint32_t rs[D];
+  const int nk = (K + kGK - 1) / kGK;
+  auto load_a = [&](int kt, u32x4_t (&qa)[4]) {
+    const int ko = min(min(kt, nk - 1) * kGK, K - 8 - pc);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      ra[i] = aok ? *reinterpret_cast<const u32x4_t*>(arow[i] + ko) : z4;
-    if (FP4) {
-      const bool cok = ko + 32 * half < K;
-      rc = cok ? *reinterpret_cast<const u32x4_t*>(crow + ko / 2) : z4;
-      rs = cok ? srow[ko / 32] : 127u;
+    for (int i = 0; i < 4; ++i) qa[i] = *reinterpret_cast<const u32x4_t*>(arow[i] + ko);
+  };
+  auto load_w = [&](int kt, u32x4_t (&qw)[FP4 ? 1 : 4], uint32_t& qs) {
+    if constexpr (FP4) {
+      const int ko = min(min(kt, nk - 1) * kGK, K - 32 - 32 * half);
+      qw[0] = *reinterpret_cast<const u32x4_t*>(crow + ko / 2);
+      qs = srow[ko / 32];
     } else {
+      const int ko = min(min(kt, nk - 1) * kGK, K - 8 - pc);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        rw[i] = aok ? *reinterpret_cast<const u32x4_t*>(wrow[i] + ko) : z4;
+      for (int i = 0; i < 4; ++i) qw[i] = *reinterpret_cast<const u32x4_t*>(wrow[i] + ko);
     }
   };
-  load_step(0);
   f32x16_t acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -321,52 +325,91 @@ __global__ __launch_bounds__(256) void k_gemm(GemmParams p) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.0f;
 
-  const int nk = (K + kGK - 1) / kGK;
-  // registers -> LDS buffer `buf`
-#define GEMM_STAGE(buf)                                                                 \
-  do {                                                                                  \
-    for (int i = 0; i < 4; ++i)                                                         \
-      *reinterpret_cast<u32x4_t*>(&As[buf][((tid + 256 * i) >> 3) * kGS + pc]) = ra[i]; \
-    if (FP4) {                                                                          \
-      u32x4_t lo, hi;                                                                   \
-      uint16_t* d = &Ws[buf][(tid >> 1) * kGS + half * 32];                             \
-      fp4x16_to_bf16(u32x2_t{rc.x, rc.y}, rs, lo, hi);                                  \
-      *reinterpret_cast<u32x4_t*>(d) = lo;                                              \
-      *reinterpret_cast<u32x4_t*>(d + 8) = hi;                                          \
-      fp4x16_to_bf16(u32x2_t{rc.z, rc.w}, rs, lo, hi);                                  \
-      *reinterpret_cast<u32x4_t*>(d + 16) = lo;                                         \
-      *reinterpret_cast<u32x4_t*>(d + 24) = hi;                                         \
-    } else {                                                                            \
-      for (int i = 0; i < 4; ++i)                                                       \
-        *reinterpret_cast<u32x4_t*>(&Ws[buf][((tid + 256 * i) >> 3) * kGS + pc]) = rw[i]; \
-    }                                                                                   \
-  } while (0)
-  GEMM_STAGE(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) load_step((kt + 1) * kGK);  // next step's loads before this step's math
+  // registers of step kt -> LDS buffer `buf`
+  const u32x4_t z4 = {0u, 0u, 0u, 0u};
+  auto stage = [&](int kt, int buf, const u32x4_t (&qa)[4], const u32x4_t (&qw)[FP4 ? 1 : 4], uint32_t qs) {
+    const bool in = kt * kGK + pc < K;
 #pragma unroll
-    for (int ks = 0; ks < kGK / 16; ++ks) {
-      bf16x8_t af[2], bf[2];
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x4_t*>(&As[buf][((tid + 256 * i) >> 3) * kGS + pc]) = in ? qa[i] : z4;
+    if constexpr (FP4) {
+      const bool win = kt * kGK + 32 * half < K;
+      const u32x4_t c = win ? qw[0] : z4;
+      const uint32_t s = win ? qs : 127u;
+      u32x4_t lo, hi;
+      uint16_t* d = &Ws[buf][(tid >> 1) * kGS + half * 32];
+      fp4x16_to_bf16(u32x2_t{c.x, c.y}, s, lo, hi);
+      *reinterpret_cast<u32x4_t*>(d) = lo;
+      *reinterpret_cast<u32x4_t*>(d + 8) = hi;
+      fp4x16_to_bf16(u32x2_t{c.z, c.w}, s, lo, hi);
+      *reinterpret_cast<u32x4_t*>(d + 16) = lo;
+      *reinterpret_cast<u32x4_t*>(d + 24) = hi;
+    } else {
 #pragma unroll
-      for (int im = 0; im < 2; ++im)
-        af[im] = *reinterpret_cast<const bf16x8_t*>(
-            &As[cur][(wm * 64 + im * 32 + (lane & 31)) * kGS + ks * 16 + 8 * (lane >> 5)]);
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<u32x4_t*>(&Ws[buf][((tid + 256 * i) >> 3) * kGS + pc]) = in ? qw[i] : z4;
+    }
+  };
+  // LDS written before it is read after it; the loads stay on their way
+  auto barrier = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
 #pragma unroll
-      for (int in = 0; in < 2; ++in)
-        bf[in] = *reinterpret_cast<const bf16x8_t*>(
-            &Ws[cur][(wn * 64 + in * 32 + (lane & 31)) * kGS + ks * 16 + 8 * (lane >> 5)]);
+  for (int d = 0; d < D; ++d) {
+    load_a(d, ra[d]);
+    load_w(d, rw[d], rs[d]);
+  }
+  stage(0, 0, ra[0], rw[0], rs[0]);
+  barrier();
+  // the K loop of a wave with nblk 32-row blocks that hold rows: a block past
+  // the tile's rows is not multiplied (nothing of it is stored); of 333 prompt
+  // rows an expert of 32 has ~42 of a tile's 128
+  auto kloop = [&](auto nblk) {
+    constexpr int NB = decltype(nblk)::value;
+    auto multiply = [&](int buf) {
 #pragma unroll
-      for (int im = 0; im < 2; ++im)
+      for (int ks = 0; ks < (NB ? kGK / 16 : 0); ++ks) {
+        bf16x8_t af[2], bf[2];
+#pragma unroll
+        for (int im = 0; im < NB; ++im)
+          af[im] = *reinterpret_cast<const bf16x8_t*>(
+              &As[buf][(wm * 64 + im * 32 + (lane & 31)) * kGS + ks * 16 + 8 * (lane >> 5)]);
 #pragma unroll
         for (int in = 0; in < 2; ++in)
-          acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[im], bf[in], acc[im][in], 0, 0, 0);
+          bf[in] = *reinterpret_cast<const bf16x8_t*>(
+              &Ws[buf][(wn * 64 + in * 32 + (lane & 31)) * kGS + ks * 16 + 8 * (lane >> 5)]);
+#pragma unroll
+        for (int im = 0; im < NB; ++im)
+#pragma unroll
+          for (int in = 0; in < 2; ++in)
+            acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[im], bf[in], acc[im][in], 0, 0, 0);
+      }
+    };
+    int kt = 0;
+    for (; kt + D <= nk; kt += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        load_a(kt + d + D, ra[d]);
+        load_w(kt + d + D, rw[d], rs[d]);
+        multiply(d & 1);
+        stage(kt + d + 1, (d + 1) & 1, ra[(d + 1) % D], rw[(d + 1) % D], rs[(d + 1) % D]);
+        barrier();
+      }
     }
-    if (kt + 1 < nk) GEMM_STAGE(cur ^ 1);
-    __syncthreads();
-  }
-#undef GEMM_STAGE
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)  // the last nk % D steps, loaded already
+      if (kt + d < nk) {
+        multiply(d & 1);
+        stage(kt + d + 1, (d + 1) & 1, ra[d + 1], rw[d + 1], rs[d + 1]);
+        barrier();
+      }
+  };
+  const int live = (rows - wm * 64 + 31) / 32;  // <= 0: no rows for this wave
+  if (live >= 2) kloop(std::integral_constant<int, 2>{});
+  else if (live == 1) kloop(std::integral_constant<int, 1>{});
+  else kloop(std::integral_constant<int, 0>{});
 
   gemm_epi_stage<MODE>(ep, epl);
   gemm_epilogue<MODE, GROUPED>(acc, p, lane, wm, wn, n0, r0, rows, ep, epl);

@@ -137,6 +137,34 @@ def test_moe_prefill_drops_out_of_range_ids(orc):
     assert rel < 2e-2
 
 
+@pytest.mark.parametrize("H,I", [(32, 96), (128, 224), (288, 320), (256, 544)])
+def test_moe_prefill_tile_edges(orc, H, I):
+    """The FP4 GEMM tiles where they can go wrong: experts of 0 to 129 rows
+    (32-row blocks of a 128-row tile that are full, partly full or skipped) and
+    K of 1 to 9 steps of 64 (whole and half last steps; every remainder of the
+    4 steps in flight).  The bars of test_moe_prefill_vs_oracle."""
+    E, k = 8, 1
+    counts = [0, 1, 31, 32, 33, 64, 97, 129]
+    M = sum(counts)
+    d = moe_weights(orc, E, H, I, seed=7)
+    x = orc.fill_bf16(7, 51, M * H, 0.0, 1.0)
+    idx = np.repeat(np.arange(E, dtype=np.int32), counts).reshape(M, 1)
+    idx = np.ascontiguousarray(idx[np.random.default_rng(7).permutation(M)])
+    score = np.ones((M, 1), np.float32)
+    want = orc.moe_experts(x, idx, score, d["guc"], d["gus"], d["gub"], d["dnc"], d["dns"],
+                           d["dnb"], E, H, I, k)
+    h = to_dev(np.zeros((M, H), np.uint16))
+    dv = {n: to_dev(v) for n, v in d.items()}
+    ne.moe_prefill(to_dev(x), to_dev(idx), to_dev(score), dv["guc"], dv["gus"], dv["gub"],
+                   dv["dnc"], dv["dns"], dv["dnb"], h, M, E, H, I, k)
+    got = orc.bf16_to_f32(to_host(h)).astype(np.float64).reshape(M, H)
+    r = orc.bf16_to_f32(want).astype(np.float64).reshape(M, H)
+    err = np.abs(got - r)
+    say(f"moe_prefill H={H} I={I}: max error / max|ref| = {err.max() / np.abs(r).max():.3e}")
+    assert err.max() < 2e-2 * np.abs(r).max()
+    assert np.median(err) <= 2.0 ** -8 * np.sqrt((r ** 2).mean())
+
+
 @pytest.mark.parametrize("window", [0, 64])
 def test_attn_prefill_vs_oracle(orc, window):
     M, Hq, Hkv, D, T = 200, 8, 2, 64, 256
