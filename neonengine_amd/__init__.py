@@ -164,6 +164,10 @@ def config_preset(name: str = "gpt-oss-20b", **overrides) -> Config:
     return cfg
 
 
+# The smallest calls are bound by this file: an attention step over a window is a
+# 5.2 us kernel under a 10.5 us wrapper when each pointer is boxed, the device
+# looked for and the workspace sized on every call, and 9.2 us as it stands.
+# Every entry point has its argtypes, so a plain int passes as a pointer whole.
 def _ptr(t):
     """Device pointer of a torch tensor (None -> NULL)."""
     if t is None:
@@ -171,7 +175,7 @@ def _ptr(t):
     if hasattr(t, "data_ptr"):
         if not t.is_contiguous():
             raise ValueError("tensor must be contiguous")
-        return C.c_void_p(t.data_ptr())
+        return t.data_ptr()
     return C.c_void_p(int(t))
 
 
@@ -182,15 +186,22 @@ def _nbytes(t):
     return t.numel() * t.element_size()
 
 
+_cuda = None  # torch.cuda once a device was found (a process does not lose it again)
+
+
 def _stream(stream):
+    """Stream handle (None -> torch's current stream, or the default one)."""
+    global _cuda
     if stream is None:
         try:
-            import torch
-            if torch.cuda.is_available():
-                return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+            if _cuda is None:
+                import torch
+                if not torch.cuda.is_available():
+                    return None
+                _cuda = torch.cuda
+            return _cuda.current_stream().cuda_stream
         except Exception:
-            pass
-        return None
+            return None
     if hasattr(stream, "cuda_stream"):
         return C.c_void_p(stream.cuda_stream)
     return C.c_void_p(int(stream))
@@ -295,11 +306,12 @@ def attn_decode_workspace(B, Hq, Hkv, D, T_max, window):
 def attn_decode(q, k_cache, v_cache, sinks, pos, out, B, Hq, Hkv, D, T_max, window,
                 stream=None, workspace=None, counters=None):
     """counters: zero-filled once by the caller (each call leaves it zero)."""
-    wb, cb = attn_decode_workspace(B, Hq, Hkv, D, T_max, window)
-    if workspace is None and wb:
-        workspace = _workspace(wb)
-    if counters is None:
-        counters = _workspace(cb, zero=True)
+    if workspace is None or counters is None:
+        wb, cb = attn_decode_workspace(B, Hq, Hkv, D, T_max, window)
+        if workspace is None and wb:
+            workspace = _workspace(wb)
+        if counters is None:
+            counters = _workspace(cb, zero=True)
     _check(lib().neon_attn_decode(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(sinks),
                                   _ptr(pos), _ptr(out), B, Hq, Hkv, D, T_max, window,
                                   _ptr(workspace), _nbytes(workspace), _ptr(counters),
