@@ -67,7 +67,7 @@ class Engine {
     check(neon_load_tensor(ctx_, name.c_str(), data, bytes), ctx_);
   }
 
-  // Prompt mode: NEON_PREFILL_CHUNKED (16 prompt rows per pass, default),
+  // Prompt mode: NEON_PREFILL_CHUNKED (up to 512 prompt rows per pass, default),
   // NEON_PREFILL_STEPWISE (every prompt token as a decode step), both
   // bit-identical; or NEON_PREFILL_BATCHED (all prompt rows at once on the
   // matrix cores, equal to the others up to bf16 rounding).

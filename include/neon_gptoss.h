@@ -92,9 +92,10 @@ neon_status neon_load_tensor(neon_ctx* ctx, const char* name,
  * the prompt; afterwards the first generated token of each sequence is
  * available.  Modes (neon_set_prefill_mode):
  *  - NEON_PREFILL_CHUNKED (default): prompt rows 0 .. n_tokens-2 of a
- *    sequence go through every layer 16 rows at a time with the batched decode
- *    kernels (each weight row read once per 16 rows, causal attention over the
- *    sequence's cache), then the last prompt token runs as a decode step.
+ *    sequence go through every layer up to 512 rows at a time (each weight row
+ *    read once per pass, causal attention over the sequence's cache; fewer than
+ *    24 rows go 16 at a time through the batched decode kernels), then the last
+ *    prompt token runs as a decode step.
  *    Bit-identical to NEON_PREFILL_STEPWISE.
  *  - NEON_PREFILL_STEPWISE: every prompt token as a decode step.
  *  - NEON_PREFILL_BATCHED: all prompt rows of a sequence at once on the

@@ -437,7 +437,7 @@ class Engine:
         self._chk(lib().neon_set_decode_mode(self._ctx, mode))
 
     def set_prefill_mode(self, mode: int):
-        """PREFILL_CHUNKED (default: 16 prompt rows per pass), PREFILL_STEPWISE
+        """PREFILL_CHUNKED (default: up to 512 prompt rows per pass), PREFILL_STEPWISE
         (every prompt token as a decode step) or PREFILL_BATCHED (all prompt rows at
         once on the matrix cores; equal to the others up to bf16 rounding)."""
         self._chk(lib().neon_set_prefill_mode(self._ctx, mode))
