@@ -17,6 +17,7 @@
 // own the units u = 16 g + b, so a lane reads its own row's units straight
 // from the stored row (256 contiguous bytes per row and group).
 #include "neon_common.hpp"
+#include "neon_exact_index.hpp"
 #include "neon_internal.hpp"
 
 namespace neon {
@@ -94,14 +95,6 @@ __device__ constexpr int xm_order(int o) {
 template <int NG>
 constexpr int xm_depth() { return NG == 6 ? 3 : NG == 8 ? 4 : NG == 4 ? 2 : NG; }
 
-// Place of element j of an act row: the 16-byte pieces of a group's units are
-// stored piece by piece ([piece][unit]), so that the 16 lanes of an input row
-// read 256 contiguous bytes per load.
-__device__ __forceinline__ int xm_act_at(int j, int U) {
-  const int g = j >> 9, b = (j >> 5) & 15, q = (j >> 3) & 3;
-  return (g << 9) + (q * min(16, U - 16 * g) + b) * 8 + (j & 7);
-}
-
 // one work item of a wave: its first row's codes and scales (uniform) and the
 // lane's input row; row quads from `quads` on re-read quad 0 (past the matrix)
 struct XmItem {
@@ -136,10 +129,10 @@ struct XmStream {
   }
   __device__ __forceinline__ void input(const XmItem& it, int o, int U, int lane) {
     asm volatile("" : "+v"(lane));
-    const int g = xm_order<NG>(o), nb = min(16, U - 16 * g);
-    const uint4* p = reinterpret_cast<const uint4*>(it.x) + 64 * g + min(lane >> 2, nb - 1);
+    const XmPieces at = xm_pieces(xm_order<NG>(o), lane >> 2, U);
+    const uint4* p = reinterpret_cast<const uint4*>(it.x) + at.first;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) x[o % D][q] = p[q * nb];
+    for (int q = 0; q < 4; ++q) x[o % D][q] = p[q * at.step];
   }
   __device__ __forceinline__ void start(const XmItem& it, int U, int lane) {
 #pragma unroll
@@ -489,11 +482,6 @@ __global__ __launch_bounds__(64 * kXmDnWaves, 1) void k_xm_down(
     const size_t o = (size_t)bb * H + n;
     out[o] = residual ? f2bf(__fadd_rn(bf2f(residual[o]), bf2f(m))) : m;
   }
-}
-
-static int xm_groups(int K) {
-  const int ng = (K / 32 + 15) / 16;
-  return ng <= 1 ? 1 : ng <= 2 ? 2 : ng <= 4 ? 4 : ng <= 6 ? 6 : ng <= 8 ? 8 : 0;
 }
 
 bool xm_moe_wanted(int B, int k, int E) {
