@@ -1313,15 +1313,18 @@ __device__ __forceinline__ float block_max_1024(float v, float* red) {
 
 // Bound: one block per row re-reads the row's e_i (804 KB at the gpt-oss
 // vocabulary, from L2) for every bit of the search, so it is the block's load
-// rate.  kSampleReg values per thread stay in registers and the others are
-// requested eight at a time; a bit whose threshold lies above every e_i or
+// rate.  REG values per thread stay in registers and the others are requested
+// eight at a time; a bit whose threshold lies above every e_i or
 // below all of them needs no pass (its sum is 0, or Z itself); the running
 // sums read the slices through LDS instead of a cache line per lane, and the
 // slice with the target is walked from LDS.  Every sum keeps its order.
-// V = 201088, top_p 0.95: 935 -> 350 us.
-constexpr int kSampleReg = 64;
+// V = 201088, top_p 0.95: 860 -> 345 us.
+// With a few values per thread (REG <= 8, which then hold the whole row) the
+// passes are short and what is left is barriers and the serial prefix: no
+// extremes, no staging, each thread reads its own slice.
 constexpr int kSampleTile = 16;  // elements of 512 slices staged at once
 
+template <int REG>
 __global__ __launch_bounds__(1024) void k_sample(
     const float* __restrict__ logits, int V, float inv_temp, float top_p, uint64_t seed,
     int32_t* __restrict__ pos, float* __restrict__ scratch, int32_t* __restrict__ out_ids,
@@ -1329,32 +1332,35 @@ __global__ __launch_bounds__(1024) void k_sample(
     int advance, int row0) {
   __shared__ float red[16];
   __shared__ __align__(16) float scan[1024];
-  __shared__ float tile[512 * (kSampleTile + 1)];
+  constexpr bool kShort = REG <= 8;  // the row is in registers: V <= 1024 REG
+  __shared__ float tile[kShort ? 1 : 512 * (kSampleTile + 1)];
   __shared__ int32_t pick, owner;
   const int b = blockIdx.x, tid = threadIdx.x;
   const float* l = logits + (size_t)b * V;
   float* e = scratch + (size_t)b * V;
   const int p = pos[b];
+  constexpr int ML = kShort ? REG : 8;
   float m = -INFINITY;
-  for (int i = tid; i < V; i += 8192) {
-    float v[8];
+  for (int i = tid; i < V; i += 1024 * ML) {
+    float v[ML];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = l[min(i + 1024 * q, V - 1)];
+    for (int q = 0; q < ML; ++q) v[q] = l[min(i + 1024 * q, V - 1)];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) m = fmaxf(m, v[q]);
+    for (int q = 0; q < ML; ++q) m = fmaxf(m, v[q]);
   }
   m = block_max_1024(m, red);
   // e_i to scratch; the thread's first values (i = tid + 1024 k) stay here, -1
   // where there is none
-  float er[kSampleReg];
+  constexpr int NB = REG < 8 ? REG : 8;  // requested at once
+  float er[REG];
   float z = 0.0f, lowest = INFINITY, highest = 0.0f;
 #pragma unroll
-  for (int k0 = 0; k0 < kSampleReg; k0 += 8) {
-    float v[8];
+  for (int k0 = 0; k0 < REG; k0 += NB) {
+    float v[NB];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = l[min(tid + 1024 * (k0 + q), V - 1)];
+    for (int q = 0; q < NB; ++q) v[q] = l[min(tid + 1024 * (k0 + q), V - 1)];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < NB; ++q) {
       const int i = tid + 1024 * (k0 + q);
       er[k0 + q] = -1.0f;
       if (i < V) {
@@ -1367,7 +1373,7 @@ __global__ __launch_bounds__(1024) void k_sample(
       }
     }
   }
-  for (int i0 = tid + 1024 * kSampleReg; i0 < V; i0 += 8192) {
+  for (int i0 = tid + 1024 * REG; !kShort && i0 < V; i0 += 8192) {
     float v[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) v[q] = l[min(i0 + 1024 * q, V - 1)];
@@ -1384,22 +1390,24 @@ __global__ __launch_bounds__(1024) void k_sample(
     }
   }
   z = block_sum_1024(z, red);  // also orders the e[] stores before the reads below
-  highest = block_max_1024(highest, red);
-  lowest = -block_max_1024(-lowest, red);
   uint32_t t_bits = 0;          // threshold as positive-float bits (0: keep all)
   float kept = z;
   if (top_p < 1.0f) {
     const float goal = __fmul_rn(top_p, z);
+    if constexpr (!kShort) {
+      highest = block_max_1024(highest, red);
+      lowest = -block_max_1024(-lowest, red);
+    }
     for (int bit = 30; bit >= 0; --bit) {
       const uint32_t cand = t_bits | (1u << bit);
       const float t = __builtin_bit_cast(float, cand);
       float s = 0.0f;
-      if (t <= lowest) {
+      if (!kShort && t <= lowest) {
         s = z;                 // every value kept
-      } else if (!(t > highest)) {
+      } else if (kShort || !(t > highest)) {
 #pragma unroll
-        for (int k = 0; k < kSampleReg; ++k) s = __fadd_rn(s, er[k] >= t ? er[k] : 0.0f);
-        for (int i0 = tid + 1024 * kSampleReg; i0 < V; i0 += 8192) {
+        for (int k = 0; k < REG; ++k) s = __fadd_rn(s, er[k] >= t ? er[k] : 0.0f);
+        for (int i0 = tid + 1024 * REG; !kShort && i0 < V; i0 += 8192) {
           float v[8];
 #pragma unroll
           for (int q = 0; q < 8; ++q) v[q] = e[min(i0 + 1024 * q, V - 1)];
@@ -1423,7 +1431,14 @@ __global__ __launch_bounds__(1024) void k_sample(
   // [tid C, tid C + C) of kept values; block prefix over the threads
   const int C = (V + 1023) / 1024;
   float local = 0.0f;
-  for (int half = 0; half < 2; ++half)
+  float es[kShort ? REG : 1];  // the thread's slice
+  if constexpr (kShort) {
+#pragma unroll
+    for (int k = 0; k < REG; ++k) es[k] = k < C && tid * C + k < V ? e[tid * C + k] : -1.0f;
+#pragma unroll
+    for (int k = 0; k < REG; ++k) local = __fadd_rn(local, es[k] >= t ? es[k] : 0.0f);
+  }
+  for (int half = 0; !kShort && half < 2; ++half)
     for (int k0 = 0; k0 < C; k0 += kSampleTile) {
       float v[8];
 #pragma unroll
@@ -1472,8 +1487,22 @@ __global__ __launch_bounds__(1024) void k_sample(
   // differently from the prefix, so the walk ends on the slice's last kept
   // index if it does not cross the target
   if (scan[tid] <= target && local > 0.0f && __fadd_rn(scan[tid], local) > target) owner = tid;
+  if constexpr (kShort) {
+    if (owner == tid) {  // written by this thread, if by any
+      float run = scan[tid];
+      int last = -1, found = -1;
+#pragma unroll
+      for (int k = 0; k < REG; ++k)
+        if (found < 0 && es[k] >= t) {
+          last = tid * C + k;
+          run = __fadd_rn(run, es[k]);
+          if (run > target) found = last;
+        }
+      pick = found >= 0 ? found : last;
+    }
+  }
   __syncthreads();
-  if (owner >= 0) {
+  if (!kShort && owner >= 0) {
     const int i0 = min(owner * C, V), i1 = min(i0 + C, V);
     float run = scan[owner];
     int last = -1, found = -1;
@@ -1518,9 +1547,22 @@ void launch_sample(const float* logits, int B, int V, float temperature, float t
                    uint64_t seed, int32_t* pos, float* scratch, int32_t* out_ids,
                    int32_t* tokens, int tok_stride, const int32_t* prompt_len, bool advance,
                    hipStream_t st, int row0) {
-  hipLaunchKernelGGL(k_sample, dim3(B), dim3(1024), 0, st, logits, V, 1.0f / temperature,
-                     top_p, seed, pos, scratch, out_ids, tokens, tok_stride, prompt_len,
-                     advance ? 1 : 0, row0);
+#define SAMPLE(REG)                                                                        \
+  hipLaunchKernelGGL(k_sample<REG>, dim3(B), dim3(1024), 0, st, logits, V, 1.0f / temperature, \
+                     top_p, seed, pos, scratch, out_ids, tokens, tok_stride, prompt_len,   \
+                     advance ? 1 : 0, row0)
+  // Every value of REG that a row does not have costs a place in each pass.  us at
+  // top_p 0.95 (1.0), one row, REG as chosen / 64 / one load per value and pass:
+  // V = 1000 22.9 (11.3) / 52.7 (17.5) / 23.7 (12.3); 4096 26.7 (13.2) / 54.9 (18.3) /
+  // 34.0 (14.8); 8192 32.0 (16.9) / 55.4 (19.1) / 57.0 (18.2); 16384 36.3 (18.4) /
+  // 57.2 (20.7) / 92.5 (24.7); 32768 48.2 (23.8) / 61.9 (25.4) / 160 (37.0).
+  if (V <= 1024) SAMPLE(1);
+  else if (V <= 4096) SAMPLE(4);
+  else if (V <= 8192) SAMPLE(8);
+  else if (V <= 16384) SAMPLE(16);
+  else if (V <= 32768) SAMPLE(32);
+  else SAMPLE(64);
+#undef SAMPLE
 }
 
 // ===========================================================================

@@ -62,6 +62,29 @@ def test_sample_bit_exact_vs_oracle(orc):
     say(f"{total} draws identical to the oracle")
 
 
+@pytest.mark.parametrize("V", [1, 64, 1024, 1025, 4096, 4097, 8192, 8193, 16384, 16385, 32768,
+                               32769, 65537])
+def test_sample_bit_exact_at_form_edges(orc, V):
+    """The first and last vocabulary of each form of the kernel (1, 4, 8, 16, 32
+    or 64 values of a thread in registers; the row whole or in part)."""
+    torch_cuda()
+    rng = np.random.default_rng(V)
+    B = 6
+    lg = (rng.normal(size=(B, V)) * rng.uniform(0.5, 4.0, (B, 1))).astype(np.float32)
+    lg[1, rng.integers(0, V, V // 3 + 1)] = lg[1, 0]  # ties
+    lg[2] = 0.0                                       # flat: every value at the threshold
+    lg[3, : V // 2] = -np.inf                         # masked half
+    lg[4, V - 1] = 40.0                               # all the weight on the last index
+    dl = to_dev(lg)
+    for temperature, top_p in ((0.7, 0.9), (1.5, 1.0), (1.0, 0.3)):
+        for seed in (3, 2 ** 41):
+            pos = rng.integers(0, 30000, B).astype(np.int32)
+            out = empty_dev((B,), np.int32)
+            ne.sample_logits(dl, B, V, temperature, top_p, seed, to_dev(pos), out)
+            want = orc.sample(lg, temperature, top_p, seed, pos)
+            assert np.array_equal(to_host(out), want), (temperature, top_p, seed)
+
+
 def test_engine_sampled_steps_match_oracle(orc):
     """The context's sampled steps (neon_set_sampling): each step's fp32
     logits are the exact path's, and the id drawn from them at the row's
