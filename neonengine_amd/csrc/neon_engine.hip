@@ -11,6 +11,7 @@
 // ABI; failures come back as neon_status with text in neon_last_error.
 #include "../../include/neon_gptoss.h"
 #include "neon_common.hpp"
+#include "neon_exact_routes.hpp"
 #include "neon_internal.hpp"
 
 #include <algorithm>
@@ -733,17 +734,11 @@ static void enqueue_rows(neon_ctx* ctx, int B, const int32_t* pos, const int32_t
     o.mode = 1; o.W = w.wo; o.bias = w.bo; o.x = ctx->attn_out; o.y = ctx->h;
     o.N = H; o.K = c.n_heads * D; o.B = B;
     o.nblk = gemv_default_grid(o.N, o.mode);
-    // more than one (row, slot) pair per expert: the top-k runs once per row
-    // before the experts, which then group the rows by expert (each used
-    // expert's weights read once); up to one, the expert kernels choose from the
-    // logits themselves, pair by pair: few pairs share an expert, and a second
-    // read of one comes from the Infinity Cache.  ms per step, grouped / pair by
-    // pair: 32 experts (12 layers) B = 2 0.956 / 0.864, 4 1.274 / 1.200, 8 1.991 /
-    // 1.835, all rows alike 4 1.152 / 1.177, 8 1.800 / 1.805, 10 2.271 / 2.393;
-    // 128 experts (8 layers) B = 2 0.814 / 0.714, 8 1.705 / 1.528, 16 3.018 / 2.741
-    const int pairs = B * c.top_k;
-    const bool grouped = B >= 2 && ((pairs <= 64 && pairs > c.n_experts) ||
-                                    xm_moe_wanted(B, c.top_k, c.n_experts));
+    // where rows that chose the same expert share its rows (neon_exact_routes.hpp)
+    // the top-k runs once per row before the experts; else the expert kernels
+    // choose from the logits themselves, pair by pair
+    const bool on_matrix = xm_moe_wanted(B, c.top_k, c.n_experts, H, c.intermediate);
+    const bool grouped = on_matrix || moe_grouped_wanted(B, c.top_k, c.n_experts, c.intermediate);
     RouterArgs r;
     r.x = ctx->h; r.norm_w = w.mlp_norm; r.eps = c.rms_eps; r.xn_out = ctx->xn;
     r.W = w.router_w; r.bias = w.router_b; r.lg_out = ctx->router_lg;
@@ -770,8 +765,8 @@ static void enqueue_rows(neon_ctx* ctx, int B, const int32_t* pos, const int32_t
     m.residual = ctx->h; m.out = ctx->h; m.B = B; m.H = H; m.I = c.intermediate;
     m.k = c.top_k; m.alpha = c.swiglu_alpha; m.limit = c.swiglu_limit; m.err = ctx->dev_err;
     m.sync = sync;
-    if (grouped && xm_moe_supported(m)) launch_xm_moe(m, st);
-    else if (grouped && moe_batched_supported(m)) launch_moe_batched(m, st);
+    if (on_matrix && xm_moe_supported(m)) launch_xm_moe(m, st);
+    else if (grouped) launch_moe_batched(m, st);
     else launch_moe(m, st);
   }
 }
@@ -2004,7 +1999,7 @@ extern "C" neon_status neon_moe_experts(
   m.out = out; m.B = B; m.H = H; m.I = I; m.k = k; m.alpha = alpha; m.limit = limit;
   m.err = device_status_word();
   if (xm_moe_supported(m)) launch_xm_moe(m, S(stream));
-  else if (moe_batched_supported(m)) launch_moe_batched(m, S(stream));
+  else if (moe_grouped_wanted(B, k, E, I)) launch_moe_batched(m, S(stream));
   else launch_moe(m, S(stream));
   KLAUNCHED();
 }

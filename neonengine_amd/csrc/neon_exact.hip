@@ -18,6 +18,7 @@
 // from the stored row (256 contiguous bytes per row and group).
 #include "neon_common.hpp"
 #include "neon_exact_index.hpp"
+#include "neon_exact_routes.hpp"
 #include "neon_internal.hpp"
 
 namespace neon {
@@ -266,6 +267,7 @@ struct XmStream {
 // ===========================================================================
 constexpr int kXmGuRq = 3;     // row quads per gate_up task
 constexpr int kXmGuTasks = 3;  // tasks per wave
+static_assert(kXmGuColumns == 2 * kXmGuRq * 4 * kXmGuTasks, "columns of a block");
 
 // LDS written and read across the waves of a block: the loads on their way
 // stay on their way (a full fence would wait for them)
@@ -484,17 +486,13 @@ __global__ __launch_bounds__(64 * kXmDnWaves, 1) void k_xm_down(
   }
 }
 
-bool xm_moe_wanted(int B, int k, int E) {
-  return B >= 2 && (int64_t)B * k <= kXmMaxPairs && 2 * B * k >= 3 * E;
-}
 bool xm_moe_supported(const MoeArgs& a) {
-  return xm_moe_wanted(a.B, a.k, a.E) && a.idx != nullptr && a.score != nullptr &&
-         a.router_lg == nullptr && a.E <= 256 && xm_groups(a.H) != 0 && xm_groups(a.I) != 0;
+  return xm_moe_wanted(a.B, a.k, a.E, a.H, a.I) && a.idx != nullptr && a.score != nullptr &&
+         a.router_lg == nullptr && xm_groups(a.H) != 0 && xm_groups(a.I) != 0;
 }
 
 void launch_xm_moe(const MoeArgs& a, hipStream_t st) {
-  const int gu_task = 2 * kXmGuRq * 4 * kXmGuTasks;  // columns per block
-  const int gu_blocks = (a.I + gu_task - 1) / gu_task;
+  const int gu_blocks = (a.I + kXmGuColumns - 1) / kXmGuColumns;
 #define GU(NG)                                                                               \
   hipLaunchKernelGGL(k_xm_gate_up<NG>, dim3(gu_blocks, a.E), dim3(256), 0, st,        \
                      a.gu_codes, a.gu_scales, a.gu_bias, a.idx, a.xn, a.act, a.B * a.k, a.H, \

@@ -262,16 +262,8 @@ void launch_mx_rope_append(const uint16_t* qkv, const int32_t* pos, const int32_
                            int key_mask, hipStream_t st);
 // 2 <= B, B k <= 64, idx / score given (router_lg NULL): each used expert's
 // weights read once for all rows that chose it; bit-identical to launch_moe
-bool moe_batched_supported(const MoeArgs& a);
 void launch_moe_batched(const MoeArgs& a, hipStream_t st);
-// the same on the fp32 matrix instructions (neon_exact.hip), at most
-// kXmMaxPairs pairs
-constexpr int kXmMaxPairs = 1280;
-// From 1.5 pairs per expert on: an instruction takes four pairs of an expert
-// whether there are four or one.  Engine steps, 20b (one pair per expert at
-// B = 8), ms, vector kernels / these: B = 4 2.46 / 2.83, 8 3.72 / 3.69, 16
-// 5.82 / 5.22, 32 11.4 / 8.22.
-bool xm_moe_wanted(int B, int k, int E);
+// the same on the fp32 matrix instructions (neon_exact.hip)
 bool xm_moe_supported(const MoeArgs& a);
 void launch_xm_moe(const MoeArgs& a, hipStream_t st);
 

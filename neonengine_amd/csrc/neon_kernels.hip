@@ -2638,9 +2638,8 @@ __global__ __launch_bounds__(1024) void k_moe_down(
 }
 
 // ===========================================================================
-// Batched experts (2 <= B, B k <= 64; few pairs per expert, see
-// xm_moe_supported for the others): rows that chose the same expert share
-// one read of its weights.  idx / score [B][k] come from the top-k kernel.
+// Batched experts (2 <= B, B k <= 64; neon_exact_routes.hpp says which calls
+// come here): rows that chose the same expert share one read of its weights.  idx / score [B][k] come from the top-k kernel.
 // Pair q = b k + s is row b's slot s; lane q of a wave holds idx[q], and
 // __ballot(idx == e) lists the pairs of expert e in row order.
 //
@@ -3223,11 +3222,6 @@ bool launch_moe_fused(const MoeArgs& a, hipStream_t st) {
     case 3: return pr ? launch_moe_fused_p<3, true>(a, st) : launch_moe_fused_p<3, false>(a, st);
     default: return false;
   }
-}
-
-bool moe_batched_supported(const MoeArgs& a) {
-  return a.B >= 2 && a.B * a.k <= 64 && a.idx != nullptr && a.score != nullptr &&
-         a.router_lg == nullptr && a.k <= kMaxTopK;
 }
 
 void launch_moe_batched(const MoeArgs& a, hipStream_t st) {

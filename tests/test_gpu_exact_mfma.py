@@ -46,9 +46,23 @@ def _run(torch, w, x, h, idx, score, E, H, I, k):
     (33, 16, 3104, 1056, 4, False), # 97 and 33 units: the first unit past 64, past 32
     (80, 4, 4096, 480, 4, True),    # 8 groups, 15 units; 20 quads of pairs per expert
     (320, 6, 64, 160, 4, False),    # the most pairs (1280)
+    # matrix form, as above but with enough column blocks to take it
+    (80, 256, 32, 32, 16, False),   # one unit per row; 256 experts, 1280 pairs
+    (160, 128, 544, 96, 4, True),   # 17 and 3 units
+    (46, 32, 4096, 480, 4, True),   # 8 groups, 15 units
+    (20, 8, 96, 2080, 4, True),     # 65 units of I: 5 groups run as 6
+    (16, 8, 320, 3104, 4, False),   # 97 units of I: 7 groups run as 8
+    (12, 32, 2880, 2880, 4, False), # the fewest rows of the 20b shape
+    (8, 8, 2880, 2880, 4, True),    # the fewest pairs: 32 of 40 column blocks
+    # grouped form
+    (9, 32, 2880, 2880, 4, True),
+    (11, 32, 2880, 2880, 4, False),
+    (10, 8, 4128, 2880, 4, True),   # rows of 129 units: past the matrix form's
+    (16, 8, 2880, 4128, 4, False),
 ])
 def test_experts_batch_bits(B, E, H, I, k, special):
-    """Rows that share experts against the same rows one at a time."""
+    """Rows that share experts against the same rows one at a time: pair by pair,
+    grouped on the vector units or on the matrix instructions, as the sizes say."""
     torch = torch_cuda()
     print(f"moe_experts B={B} E={E} H={H} I={I} k={k} special={special}", flush=True)
     w, x, h, idx, score = _experts(torch, B, E, H, I, k, 7 * B + E, special)
@@ -60,6 +74,43 @@ def test_experts_batch_bits(B, E, H, I, k, special):
             ne.device_check()
     same = (got.view(torch.int16) == ref.view(torch.int16)) | (got.isnan() & ref.isnan())
     assert bool(same.all()), int((~same).sum())
+
+
+@pytest.mark.parametrize("B", [11, 12, 13, 16])
+def test_experts_alike_bits(B):
+    """Every row on the same four experts, on both sides of the line between the
+    grouped and the matrix form."""
+    torch = torch_cuda()
+    E, H, I, k = 32, 2880, 2880, 4
+    print(f"moe_experts alike B={B}", flush=True)
+    w, x, h, idx, score = _experts(torch, B, E, H, I, k, B, False)
+    idx = idx[:1].expand(B, k).contiguous()
+    got = _run(torch, w, x, h, idx, score, E, H, I, k)
+    ref = torch.cat([_run(torch, w, x[b:b + 1], h[b:b + 1], idx[b:b + 1], score[b:b + 1], E, H, I, k)
+                     for b in range(B)])
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("B", [8, 9, 11, 12])
+def test_engine_batch_rows_bits(B):
+    """Decode steps of the 20b layer shape at the batches where the experts change
+    form (pair by pair, grouped, matrix): each row's logits are those of the
+    sequence decoding alone; half of the rows are alike."""
+    torch_cuda()
+    print(f"engine rows B={B}", flush=True)
+    cfg = ne.config_preset("gpt-oss-20b", n_layers=2, vocab=2048, max_seq=64, max_batch=12)
+    eng = ne.Engine(cfg)
+    eng.init_random(9)
+    prompts = [[(31 * i + 17 * (b // 2 if b % 4 < 2 else b) + 3) % 2048 for i in range(4)]
+               for b in range(B)]
+    eng.prefill(prompts)
+    eng.decode(3)
+    got = eng.read_logits()
+    for b in range(0, B, 3):
+        eng.prefill([prompts[b]])
+        eng.decode(3)
+        assert eng.read_logits()[0].tobytes() == got[b].tobytes(), b
+    eng.close()
 
 
 SMALL = dict(n_layers=2, hidden=512, n_heads=16, n_kv_heads=2, head_dim=64, n_experts=8, top_k=4,
