@@ -58,4 +58,29 @@ inline bool moe_grouped_wanted(int B, int k, int E, int I) {
   return pairs <= 64 && pairs > E && xm_blocks(I) >= 36 && moe_wide(B, k, E, I);
 }
 
+// ---- decode attention: B rows, Hq / Hkv heads, S key splits of a span of keys ----
+// The matrix form (k_xa_attn) costs the same for 1 and for 8 query heads per kv
+// head; the vector form (k_attn_split) has work per head and blocks that all wait
+// for a slot.  The span is the cache's rows or the window, whichever is less; how
+// many keys a row holds is not known here.  us, vector / matrix, span full (an
+// eighth full):
+//   one split (a vector block per query head):
+//     8 heads per kv head, 128 keys: B Hq = 1024 10.7 / 8.3 (10.7 / 7.7), 4096 35 / 12
+//     4: 512 6.5 / 8.2, 1024 10.7 / 8.6; 2: 1024 10.7 / 11.8, 2048 19.9 / 17.9
+//     1: 512 6.5 / 11.7, 2048 23.2 / 29.7
+//   several (a block per kv head and split):
+//     8, 2048 keys: B Hkv S = 256 8.9 / 9.0, 512 15.7 / 11.1, 2048 44.7 / 21.6;
+//     8192 keys: 256 13.3 / 15.8, 512 24.9 / 21.3, 2048 83.4 / 51.2
+//     4, 2048 keys: 512 8.7 / 10.7, 1024 14.6 / 14.2, 2048 23.8 / 21.1
+//     1, 2048 keys: 512 8.1 / 10.3, 1024 13.5 / 13.9, 2048 21.7 / 21.0, 4096 37 / 33
+//     longer splits, 2048 blocks: 4, 4096 keys 32.6 / 32.5 (17.6 / 13.2), 8192 keys
+//     44 / 51; 1, 4096 keys 30 / 32 (16.6 / 12.5), 8192 keys 41 / 51; 4096 blocks:
+//     1, 4096 keys 50 / 53 (27 / 18), 8192 keys 69 / 100 (30 / 24)
+inline bool attn_on_matrix(int B, int Hq, int Hkv, int S, int span) {
+  const int G = Hq / Hkv;
+  const int64_t heads = B * (int64_t)Hq, blocks = B * (int64_t)Hkv * S;
+  if (S == 1) return G >= 4 ? heads > 512 : G == 2 && heads >= 2048;
+  return G == 8 ? blocks >= 512 : span <= (G == 4 ? 128 : 64) * S && blocks >= 2048;
+}
+
 }  // namespace neon

@@ -9,6 +9,7 @@
 // .py, cited as HFM:<line>); the reference repository has no implementation
 // of this path.
 #include "neon_common.hpp"
+#include "neon_exact_routes.hpp"
 #include "neon_internal.hpp"
 
 #include <math.h>
@@ -3624,18 +3625,9 @@ void launch_attn_merge(const AttnArgs& a, hipStream_t st) {
                      a.sinks, a.out, a.Hq, a.S, a.out_packed);
 }
 
-// Where the matrix-instruction form takes over (the same bits): with several
-// splits from two blocks per CU on, with one split from two of this form's
-// (one per query head).  us, this form / the other, 64 / 8 heads: several
-// splits, B = 2 T = 1024 (256 blocks) 7.8 / 8.0, B = 4 T = 1024 (512) 13.8 /
-// 10.0, B = 8 T = 2048 43.3 / 21.0, B = 8 T = 8192 76.6 / 50.4; one split, 128
-// keys, B = 8 6.0 / 7.5, B = 12 9.3 / 7.6, 256 keys, B = 32 26.8 / 12.6.
-static bool attn_on_matrix(const AttnArgs& a) {
-  return a.S > 1 ? (int64_t)a.B * a.Hkv * a.S >= 512 : (int64_t)a.B * a.Hq > 512;
-}
-
 void launch_attn(const AttnArgs& a, hipStream_t st) {
-  if (attn_on_matrix(a)) {
+  const int span = a.window > 0 && a.window < a.T_max ? a.window : a.T_max;
+  if (attn_on_matrix(a.B, a.Hq, a.Hkv, a.S, span)) {
     launch_xa_attn(a, a.window > 0 ? a.window : a.T_max, st);
     return;
   }

@@ -60,6 +60,32 @@ int main() {
   MOE(320, 4, 32, 2880, 2880, MATRIX);
   MOE(321, 4, 32, 2880, 2880, PAIRS);
   MOE(65535, 16, 256, 8192, 8192, PAIRS);
+#define ATTN(B, Hq, Hkv, S, span, want) expect("attn B=" #B " heads " #Hq "/" #Hkv " S=" #S " span " #span, neon::attn_on_matrix(B, Hq, Hkv, S, span), want)
+  // one split
+  ATTN(8, 64, 8, 1, 128, 0);
+  ATTN(16, 64, 8, 1, 128, 1);
+  ATTN(64, 64, 8, 1, 256, 1);
+  ATTN(64, 16, 2, 1, 256, 1);
+  ATTN(16, 32, 8, 1, 128, 0);
+  ATTN(32, 32, 8, 1, 128, 1);
+  ATTN(64, 16, 8, 1, 128, 0);
+  ATTN(72, 16, 8, 1, 128, 0);
+  ATTN(128, 16, 8, 1, 128, 1);
+  ATTN(65, 8, 8, 1, 128, 0);
+  ATTN(256, 8, 8, 1, 128, 0);
+  // several
+  ATTN(1, 64, 8, 32, 4096, 0);
+  ATTN(2, 64, 8, 32, 4096, 1);
+  ATTN(8, 64, 8, 8, 512, 1);
+  ATTN(16, 64, 8, 32, 32768, 1);
+  ATTN(2, 8, 8, 32, 4096, 0);
+  ATTN(8, 8, 8, 8, 512, 0);
+  ATTN(8, 32, 8, 8, 512, 0);
+  ATTN(8, 32, 8, 32, 8192, 0);
+  ATTN(8, 32, 8, 32, 4096, 1);
+  ATTN(32, 8, 8, 32, 4096, 0);
+  ATTN(8, 8, 8, 32, 2048, 1);
+  ATTN(32, 32, 8, 8, 512, 1);
   std::printf("%d calls, %d on the wrong form\n", n, bad);
   return bad != 0;
 }

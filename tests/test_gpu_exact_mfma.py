@@ -154,6 +154,12 @@ def test_prompt_passes_bits(lens, over):
     (33, 16, 4, 700, 0),   # four heads, 11 splits of one chunk, most of them empty early on
     (5, 64, 8, 2200, 0),   # 32 splits of one or two chunks
     (20, 64, 8, 300, 77),  # windows that start inside a chunk
+    # the matrix form with fewer heads per kv head than columns are made for
+    (64, 8, 8, 700, 0),    # one head, 11 splits
+    (128, 16, 8, 64, 0),   # two heads, one split of one chunk
+    (48, 16, 4, 700, 0),   # four heads, 11 splits
+    (36, 16, 4, 200, 130), # four heads, one split, windows of up to 3 chunks
+    (16, 16, 4, 3000, 0),  # four heads, 32 splits of one or two chunks
 ])
 def test_attention_batch_bits(B, Hq, Hkv, T, window):
     """Batches large enough for the matrix form against one row at a time, with
