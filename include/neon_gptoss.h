@@ -91,12 +91,17 @@ neon_status neon_load_tensor(neon_ctx* ctx, const char* name,
 /* Starts `batch` sequences from host prompt ids [batch][n_tokens] and runs
  * the prompt; afterwards the first generated token of each sequence is
  * available.  Modes (neon_set_prefill_mode):
- *  - NEON_PREFILL_CHUNKED (default): prompt rows 0 .. n_tokens-2 of a
- *    sequence go through every layer up to 512 rows at a time (each weight row
- *    read once per pass, causal attention over the sequence's cache; fewer than
- *    24 rows go 16 at a time through the batched decode kernels), then the last
- *    prompt token runs as a decode step.
- *    Bit-identical to NEON_PREFILL_STEPWISE.
+ *  - NEON_PREFILL_CHUNKED (default): prompt rows 0 .. n_tokens-2 of every
+ *    sequence go through every layer up to 512 rows at a time (each expert row
+ *    read once per pass, the QKV and O weights once to be laid out and then once
+ *    per 32 rows; causal attention over the sequence's cache), then the last
+ *    prompt token runs as a decode step.  Where few rows are left (20b: fewer
+ *    than 78, 120b: 166, with fewer experts from 49 on) they go 16 at a time
+ *    through the batched decode kernels, which is faster there.  Bit-identical to
+ *    NEON_PREFILL_STEPWISE.  The first such wide pass of a context (here or in
+ *    neon_seq_add) allocates its scratch, 125 to 195 MB for the presets, which
+ *    neon_ctx_destroy frees; if the device has no memory for it then, the context
+ *    keeps to passes of 16 rows.
  *  - NEON_PREFILL_STEPWISE: every prompt token as a decode step.
  *  - NEON_PREFILL_BATCHED: all prompt rows of a sequence at once on the
  *    matrix cores (bf16 MFMA GEMMs, grouped MXFP4 expert GEMMs, tiled causal

@@ -1120,10 +1120,13 @@ extern "C" neon_status neon_set_prefill_mode(neon_ctx* ctx, int mode) {
 // the KV append and attention over xg_sub of them at a time.  Bit-identical to
 // passes of kPromptRows rows.
 // ---------------------------------------------------------------------------
-// Rows of the largest pass (a longer one fills the 16-pair expert tiles better:
-// 512 rows x 4 experts / 32 = 64 pairs each) and from which a pass runs this
-// way: fewer rows than that take the decode kernels' 16 at a time.
-constexpr int kXgRows = 512, kXgMinRows = 24;
+// Rows of the largest pass: a longer one fills the 16-pair expert tiles better
+// (512 rows x 4 experts / 32 = 64 pairs each).  Fewer rows than xg_min_rows take the
+// decode kernels' 16 at a time.
+constexpr int kXgRows = 512;
+static int64_t xg_least(const neon_config& c) {
+  return xg_min_rows(c.n_experts, c.top_k, c.hidden, c.intermediate);
+}
 
 static bool ensure_xg(neon_ctx* ctx) {
   if (ctx->xg) return true;
@@ -1133,7 +1136,7 @@ static bool ensure_xg(neon_ctx* ctx) {
   const size_t qd = (size_t)c.n_heads * c.head_dim, qr = qd + 2 * (size_t)c.n_kv_heads * c.head_dim;
   const int rows = std::min(kXgRows, kXgMaxPairs / c.top_k) / 16 * 16;
   ctx->xg_failed = true;
-  if (!xg_supported(c.hidden, c.intermediate, (int)qd, (int)qr, c.n_experts) || rows < kXgMinRows)
+  if (!xg_supported(c.hidden, c.intermediate, (int)qd, (int)qr, c.n_experts) || rows < xg_least(c))
     return false;
   // a ring cache takes the rows of one attention launch beside its window
   int sub = std::min(128, rows);
@@ -1229,9 +1232,10 @@ static void enqueue_rows_many(neon_ctx* ctx, const int32_t* pos, int R, hipStrea
 // is synchronised.
 static neon_status prompt_rows(neon_ctx* ctx, const int32_t* rp, const int32_t* rs, size_t n_rows,
                                int per, hipStream_t st) {
+  const size_t least = (size_t)xg_least(ctx->cfg);
   for (size_t r0 = 0; r0 < n_rows;) {
     const size_t left = n_rows - r0;
-    if (per > 1 && left >= (size_t)kXgMinRows && ensure_xg(ctx)) {
+    if (per > 1 && left >= least && ensure_xg(ctx)) {
       const int R = (int)std::min<size_t>(ctx->xg_rows, left);
       HIPCHK(ctx, hipMemcpyAsync(ctx->xg_pos, rp + r0, R * 4, hipMemcpyHostToDevice, st));
       HIPCHK(ctx, hipMemcpyAsync(ctx->xg_seq, rs + r0, R * 4, hipMemcpyHostToDevice, st));

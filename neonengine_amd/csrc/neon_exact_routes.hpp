@@ -83,4 +83,18 @@ inline bool attn_on_matrix(int B, int Hq, int Hkv, int S, int span) {
   return G == 8 ? blocks >= 512 : span <= (G == 4 ? 128 : 64) * S && blocks >= 2048;
 }
 
+// ---- prompt rows: the fewest of a wide pass --------------------------------------
+// A wide pass (neon_exact_prompt.hip) takes an expert's pairs 16 at a time and
+// pays for a whole tile of every expert that any row chose, so it costs about as
+// much for few rows as for many: 49 rows' worth of the passes of 16 for what does
+// not depend on the experts, and one row's more for every 2.25 million of E H I / k.
+// ms, four layers, passes of 16 / wide, H = I = 2880, top-4: E = 8 40 rows 1.91 / 2.10,
+// 64 2.87 / 2.17; E = 32 24 rows 1.54 / 3.70, 64 3.17 / 3.77, 80 3.94 / 3.91, 128
+// 6.23 / 4.44; E = 128 24 rows 2.00 / 6.86, 128 8.90 / 11.06, 160 11.07 / 11.34, 192
+// 13.2 / 11.7; E = 32 top-1 128 rows 3.49 / 3.92, 192 5.18 / 4.25; 512, 32, top-4 48
+// rows 0.67 / 0.72, 64 0.85 / 0.74; 4096, 8, top-2 64 rows 3.01 / 3.17, 80 3.75 / 3.25.
+inline int64_t xg_min_rows(int E, int k, int H, int I) {
+  return 49 + E * (int64_t)H * I / (k * (int64_t)2250000);
+}
+
 }  // namespace neon

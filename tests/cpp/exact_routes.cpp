@@ -86,6 +86,29 @@ int main() {
   ATTN(32, 8, 8, 32, 4096, 0);
   ATTN(8, 8, 8, 32, 2048, 1);
   ATTN(32, 32, 8, 8, 512, 1);
+#define WIDE(rows, E, k, H, I, want) expect(#rows " rows E=" #E " k=" #k " H=" #H " I=" #I, rows >= neon::xg_min_rows(E, k, H, I), want)
+  WIDE(24, 32, 4, 2880, 2880, 0);
+  WIDE(64, 32, 4, 2880, 2880, 0);
+  WIDE(96, 32, 4, 2880, 2880, 1);
+  WIDE(24, 128, 4, 2880, 2880, 0);
+  WIDE(128, 128, 4, 2880, 2880, 0);
+  WIDE(160, 128, 4, 2880, 2880, 0);
+  WIDE(174, 128, 4, 2880, 2880, 1);
+  WIDE(192, 128, 4, 2880, 2880, 1);
+  WIDE(80, 64, 4, 2880, 2880, 0);
+  WIDE(112, 64, 4, 2880, 2880, 1);
+  WIDE(48, 16, 4, 2880, 2880, 0);
+  WIDE(64, 16, 4, 2880, 2880, 1);
+  WIDE(40, 8, 4, 2880, 2880, 0);
+  WIDE(64, 8, 4, 2880, 2880, 1);
+  WIDE(128, 32, 1, 2880, 2880, 0);
+  WIDE(192, 32, 1, 2880, 2880, 1);
+  WIDE(48, 32, 4, 512, 512, 0);
+  WIDE(64, 32, 4, 512, 512, 1);
+  WIDE(48, 64, 6, 2048, 1408, 0);
+  WIDE(80, 64, 6, 2048, 1408, 1);
+  WIDE(64, 8, 2, 4096, 4096, 0);
+  WIDE(96, 8, 2, 4096, 4096, 1);
   std::printf("%d calls, %d on the wrong form\n", n, bad);
   return bad != 0;
 }

@@ -118,9 +118,12 @@ SMALL = dict(n_layers=2, hidden=512, n_heads=16, n_kv_heads=2, head_dim=64, n_ex
 
 
 @pytest.mark.parametrize("lens,over", [
-    ([25], {}),                                    # the fewest rows of a wide pass
+    ([25], {}),                                    # 24 rows: passes of 16 and 8
+    ([49], {}),                                    # 48 rows: the most by 16
+    ([50], {}),                                    # 49 rows: the fewest of a wide pass
     ([145], {}),                                   # a second attention launch of 16 rows
     ([530], {}),                                   # a pass of 512 rows, then 17 by 16s; ring wraps
+    ([562], {}),                                   # a pass of 512 rows, then a wide one of 49
     ([40, 3, 1, 90], {}),                          # several sequences in one pass
     ([200], dict(sliding_window=40)),              # ring of 64 rows: 24 rows per attention launch
     ([70], dict(hidden=192, intermediate=320)),    # 6 and 10 units: short rows, empty chains
