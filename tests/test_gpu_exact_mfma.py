@@ -196,8 +196,9 @@ def test_attention_batch_bits(B, Hq, Hkv, T, window):
 @pytest.mark.parametrize("V,T,p", [(1, 1.0, 0.9), (1000, 0.7, 0.9), (66560, 1.3, 0.999),
                                    (70001, 0.5, 1.0), (201088, 0.8, 0.95)])
 def test_sampling_rows_alike(V, T, p):
-    """Rows of a batch draw what they draw alone, and equal logits (every value
-    at the threshold) stay in range."""
+    """A batch draws the same ids twice, its first row (the draw's key holds the
+    row) the id that it draws alone, and equal logits (every value at the
+    threshold) stay in range."""
     torch = torch_cuda()
     print(f"sampling V={V} T={T} top_p={p}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(V)

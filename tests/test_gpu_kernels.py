@@ -315,9 +315,9 @@ def test_moe_layer_residual(orc):
 @pytest.mark.parametrize("B", [1, 4, 16, 20])
 def test_moe_experts_config0(orc, B):
     """Caller-given ids / weights (the router's) through neon_moe_experts:
-    B = 1 runs the per-row kernels, 4 and 16 the grouped kernels (each used
-    expert read once for its rows), 20 (80 pairs) the per-row kernels again;
-    all bit-identical to the canonical per-row oracle."""
+    B = 1 and 4 run the kernels that go pair by pair, 16 and 20 (two and more
+    pairs per expert) the fp32 matrix kernels; all bit-identical to the canonical
+    per-row oracle.  (The grouped vector kernels: test_experts_batch_bits.)"""
     E, H, I, k = 32, 2880, 2880, 4
     d = moe_inputs(orc, E, H, I, B, seed=4)
     _, ridx, rsc = orc.moe_layer(d["x"], d["rw"], d["rb"], d["guc"], d["gus"], d["gub"],

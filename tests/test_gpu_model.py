@@ -153,8 +153,8 @@ def test_small_model_batched_decode(orc, batch):
 
 @pytest.mark.parametrize("batch", [1, 8])
 def test_small_model_128_experts(orc, batch):
-    """E = 128 (the 120b router width): the two-quarter top-k ranking and, at
-    batch 8, the expert grouping over 128 candidate experts."""
+    """E = 128 (the 120b router width): the two-quarter top-k ranking, in the
+    expert kernels that choose from the logits themselves at either batch."""
     cfg, ocfg = pair(orc, **dict(SMALL, n_experts=128, intermediate=256, max_batch=batch,
                                  max_seq=64))
     prompt = [[(17 * i + 3 * b + 2) % 4096 for i in range(6)] for b in range(batch)]
@@ -164,8 +164,8 @@ def test_small_model_128_experts(orc, batch):
 
 
 def test_small_model_batch32(orc):
-    """Batch 32: two 16-row input blocks per projection, and the per-row expert
-    kernels (32 rows x 4 slots is past the grouped kernels' 64 pairs)."""
+    """Batch 32: two 16-row input blocks per projection, and experts that go pair
+    by pair (16 pairs each, but too few columns to share them)."""
     cfg, ocfg = pair(orc, **dict(SMALL, max_batch=32, max_seq=48))
     prompt = [[(7 * i + 5 * b + 1) % 4096 for i in range(5)] for b in range(32)]
     same, e1, e2 = run_parity(orc, cfg, ocfg, 31, prompt, 10, batch=32)
@@ -183,8 +183,8 @@ def test_gpt_oss_20b_batch4(orc):
 
 
 def test_small_model_chunked_prompt(orc):
-    """Two 40-token prompts in passes of 16, 16 and 7 rows (the last pass
-    partial), then 24 greedy steps: bit-identical to the oracle."""
+    """Two 40-token prompts, their 78 rows in one wide pass, then 24 greedy steps:
+    bit-identical to the oracle."""
     cfg, ocfg = pair(orc, **dict(SMALL, max_seq=96))
     prompt = [[(5 * i + 1) % 4096 for i in range(40)], [(9 * i + 2) % 4096 for i in range(40)]]
     same, e1, e2 = run_parity(orc, cfg, ocfg, 17, prompt, 24, batch=2, mode=ne.PREFILL_CHUNKED)
@@ -193,8 +193,8 @@ def test_small_model_chunked_prompt(orc):
 
 
 def test_small_model_sliding_ring_wraps(orc):
-    """max_seq 700: the sliding layers keep a 256-row ring (window 128 + one
-    prompt pass of 16 rows, rounded up to a power of two).  A 600-token prompt
+    """max_seq 700: the sliding layers keep a 256-row ring (window 128 + the 16
+    rows of a narrow prompt pass, rounded up to a power of two).  A 600-token prompt
     and 40 steps wrap it twice; every id and the logits must still equal the
     oracle's, which keeps every position."""
     cfg, ocfg = pair(orc, **dict(SMALL, max_seq=700, max_batch=1))
@@ -205,8 +205,8 @@ def test_small_model_sliding_ring_wraps(orc):
 
 
 def test_gpt_oss_20b_chunked_prompt(orc):
-    """20b shape, a 150-token prompt in 10 passes: the 128-key sliding window
-    moves inside the prompt."""
+    """20b shape, a 150-token prompt in one wide pass (two attention launches): the
+    128-key sliding window moves inside the prompt."""
     cfg, ocfg = pair(orc, max_seq=192)
     prompt = [[(1009 * i + 17) % 201088 for i in range(150)]]
     same, e1, e2 = run_parity(orc, cfg, ocfg, 2, prompt, 8, mode=ne.PREFILL_CHUNKED)

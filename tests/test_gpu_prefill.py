@@ -165,6 +165,52 @@ def test_moe_prefill_tile_edges(orc, H, I):
     assert np.median(err) <= 2.0 ** -8 * np.sqrt((r ** 2).mean())
 
 
+@pytest.mark.parametrize("gate,up", [(6.0, 7.0), (2.0 ** -9, 0.0)])
+def test_moe_prefill_every_scale_and_code(orc, gate, up):
+    """Every E8M0 scale (0, 1, 254 and the NaN 255 among them) times every E2M1
+    code at every place of a 32-value block, through the bf16 form's
+    dequantisation: expert e's activation is A at column e and 0 elsewhere (x is
+    0, the gate bias one-hot), its down row h holds the code of h / 256 at that
+    column and the scale h % 256, so out[e][h] is bf16(A W).  The products are
+    exact in fp32 where they are normal (8 + 2 bits); gate 6 lifts the
+    subnormal weights above 2^-126, gate 2^-9 keeps the largest finite."""
+    H, I, E = 4096, 32, 32
+    M = E
+    cols, rows = np.arange(I), np.arange(H)
+    guc = np.zeros((E, 2 * I, H // 2), np.uint8)
+    gus = np.full((E, 2 * I, H // 32), 127, np.uint8)
+    gub = np.zeros((E, 2 * I), np.float32)
+    gub[cols, 2 * cols] = gate
+    gub[:, 1::2] = up
+    dnc = np.zeros((E, H, I // 2), np.uint8)
+    for e in range(E):
+        dnc[e, :, e // 2] = (rows // 256) << (4 * (e & 1))
+    dns = np.broadcast_to((rows % 256).astype(np.uint8)[None, :, None], (E, H, 1))
+    h = to_dev(np.zeros((M, H), np.uint16))
+    say(f"moe_prefill scales x codes, gate {gate}")
+    ne.moe_prefill(to_dev(np.zeros((M, H), np.uint16)), to_dev(cols.astype(np.int32).reshape(M, 1)),
+                   to_dev(np.ones((M, 1), np.float32)), to_dev(guc), to_dev(gus),
+                   to_dev(orc.f32_to_bf16(gub)), to_dev(dnc), to_dev(dns),
+                   to_dev(np.zeros((E, H), np.uint16)), h, M, E, H, I, 1)
+    got = orc.bf16_to_f32(to_host(h)).reshape(M, H).astype(np.float64)
+    e2m1 = np.array([0, 0.5, 1, 1.5, 2, 3, 4, 6], np.float64)
+    val = np.concatenate([e2m1, -e2m1])[rows // 256]
+    w = np.ldexp(val, rows % 256 - 127)                     # exact in float64
+    w[np.abs(w) > 3.4e38] = np.copysign(np.inf, w[np.abs(w) > 3.4e38])  # 2^128 and more
+    w[rows % 256 == 255] = np.nan
+    A = got[0, 2 * 256 + 127]                               # the weight 1.0
+    assert np.isfinite(A) and A > 0 and (got[:, 2 * 256 + 127] == A).all()
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = orc.bf16_to_f32(orc.f32_to_bf16((A * w).astype(np.float32))).astype(np.float64)
+    small = (np.abs(A * w) > 0) & (np.abs(A * w) < 2.0 ** -126)  # subnormal results: not claimed
+    ok = (got == want[None, :]) | (np.isnan(got) & np.isnan(want)[None, :]) | small[None, :]
+    bad = np.argwhere(~ok)
+    assert len(bad) == 0, [(int(e), int(r) // 256, int(r) % 256, got[e, r], want[r])
+                           for e, r in bad[:8]]
+    if gate > 1:
+        assert not small.any()
+
+
 @pytest.mark.parametrize("window", [0, 64])
 def test_attn_prefill_vs_oracle(orc, window):
     M, Hq, Hkv, D, T = 200, 8, 2, 64, 256

@@ -2,8 +2,8 @@
 (neon_prefill_ragged): every sequence keeps its own position, and in the
 exact modes each sequence's fp32 logits are bit-identical to the CPU oracle
 running that sequence alone.  Prompt lengths 5, 77, 300 and 1000 cross the
-16-row chunk boundaries at different offsets, put rows of several sequences
-into one chunked pass, and wrap the sliding layers' 256-row ring cache
+boundaries of passes and of attention launches at different offsets, put rows
+of several sequences into one pass, and wrap the sliding layers' 256-row ring cache
 (1000 > 256) while the shorter sequences do not.
 """
 import sys
@@ -116,7 +116,7 @@ def test_ragged_equals_each_sequence_alone_on_gpu():
 
 def test_ragged_lengths_with_single_token_prompts(orc):
     """Prompts of 1 token (no prompt rows, only the first decode step) next to
-    longer ones, and one sequence exactly one chunk long."""
+    longer ones, and one sequence of exactly one 16-row pass."""
     cfg = ne.config_preset("gpt-oss-20b", **dict(SMALL, max_seq=64))
     seed, n_steps = 8, 5
     prompts = prompts_for((1, 17, 1, 2), cfg.vocab, 21)
