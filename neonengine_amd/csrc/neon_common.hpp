@@ -27,6 +27,25 @@ __device__ __forceinline__ uint8_t load_weight1(const uint8_t* p) {
   return __builtin_nontemporal_load(p);
 }
 
+// LDS written before it is read after it, across the waves of a block; the
+// loads on their way stay on their way (a full fence would wait for them)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+typedef float xf4 __attribute__((ext_vector_type(4)));  // accumulator of an fp32 MFMA
+
+// the values are in registers here: what makes them stays before, what uses them after
+__device__ __forceinline__ void pin4(float (&v)[4]) {
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+__device__ __forceinline__ void pin8(float (&v)[8]) {
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]),
+                    "+v"(v[6]), "+v"(v[7]));
+}
+
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

@@ -409,9 +409,10 @@ static neon_status ctx_alloc(neon_ctx* ctx) {
   // ---- KV cache ----
   // Full layers keep every position.  A sliding layer only ever reads the
   // last `window` keys, so it keeps a power-of-two ring of at least
-  // window + kPromptRows rows (a prompt pass appends kPromptRows rows before
-  // its attention reads the oldest key of its first row's window): position
-  // p lives in row p & (rows - 1).
+  // window + kPromptRows rows: position p lives in row p & (rows - 1).  An
+  // attention launch's rows are appended before it reads the oldest key of its
+  // first row's window, so it takes kPromptRows rows, or in a wide pass up to
+  // ring - window (xg_sub).
   ctx->kv_off.assign(L, 0);
   ctx->kv_rows.assign(L, c.max_seq);
   ctx->kv_mask.assign(L, -1);

@@ -23,8 +23,6 @@
 
 namespace neon {
 
-typedef float xf4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ xf4 xm_mfma(float a, float b, xf4 c) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 }
@@ -78,10 +76,6 @@ __device__ __forceinline__ float xm_fold(const float (&a)[N], int lane) {
 // 1, 5, .. 3, 7, ..: groups of one residue mod 4 hold the units l, l + 64, ..
 // of the same lanes l, off 32 pairs residues 0-2 and 1-3, off 16 their sums.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void pin8(float (&v)[8]) {
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]),
-                    "+v"(v[6]), "+v"(v[7]));
-}
 template <int NG>
 __device__ constexpr int xm_order(int o) {
   int n = 0;
@@ -268,14 +262,6 @@ struct XmStream {
 constexpr int kXmGuRq = 3;     // row quads per gate_up task
 constexpr int kXmGuTasks = 3;  // tasks per wave
 static_assert(kXmGuColumns == 2 * kXmGuRq * 4 * kXmGuTasks, "columns of a block");
-
-// LDS written and read across the waves of a block: the loads on their way
-// stay on their way (a full fence would wait for them)
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 template <int NG>
 __global__ __launch_bounds__(256, 2) void k_xm_gate_up(

@@ -30,8 +30,6 @@
 
 namespace neon {
 
-typedef float xf4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ xf4 xa_mfma(float a, float b, xf4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -55,17 +53,6 @@ __device__ __forceinline__ void xa_transpose(float (&v)[4]) {
 }
 __device__ __forceinline__ void xa_unpack(float (&v)[4], const uint2& w) {
   v[0] = bf_lo(w.x); v[1] = bf_hi(w.x); v[2] = bf_lo(w.y); v[3] = bf_hi(w.y);
-}
-
-
-__device__ __forceinline__ void pin4(float (&v)[4]) {
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
-}
-// LDS written before it is read after it, loads on their way stay on their way
-__device__ __forceinline__ void xa_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 constexpr int kXaVStride = 72;  // bf16 per key row in LDS: 16-byte rows, spread over the banks
@@ -164,7 +151,7 @@ __global__ __launch_bounds__(256, 4) void k_xa_attn(
     cm = fmaxf(cm, xor_lane<32>(cm));
     cm = fmaxf(cm, xor_lane<16>(cm));
     if (h4 == 0) lds.mx[buf][w][j] = cm;
-    xa_barrier();
+    lds_barrier();
     // ---- weights ----
     cm = fmaxf(fmaxf(lds.mx[buf][0][j], lds.mx[buf][1][j]), fmaxf(lds.mx[buf][2][j], lds.mx[buf][3][j]));
     const float mn = fmaxf(mx, cm);
@@ -179,7 +166,7 @@ __global__ __launch_bounds__(256, 4) void k_xa_attn(
     for (int kg = 0; kg < 8; ++kg)
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[kg][r] = __fmul_rn(o[kg][r], alpha);
-    xa_barrier();
+    lds_barrier();
     // pb[s2][kg]: the weight of key kg + 8 (4 s2 + kk) for lane kk; va: its V at
     // the lane's dim
     float pb[2][8], va[2][8];
@@ -217,7 +204,7 @@ __global__ __launch_bounds__(256, 4) void k_xa_attn(
                       __fadd_rn(__fadd_rn(o[4][r], o[5][r]), __fadd_rn(o[6][r], o[7][r])));
   if (ns == 1) {  // the only split with keys: the merge with the sink
     if (w == 0 && h4 == 0) lds.l[j] = l;
-    xa_barrier();
+    lds_barrier();
     l = lds.l[j];
     const float sk = bf2f(sink_raw);
     const float M = fmaxf(sk, mx);

@@ -23,8 +23,6 @@
 
 namespace neon {
 
-typedef float xf4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ xf4 xg_mfma(float a, float b, xf4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -168,11 +166,6 @@ static size_t xg_expert_lds(int U) {
   return (size_t)32 * (U | 1) * 16 + (size_t)U * 32 * 2 + (size_t)(U + 4) * 4;
 }
 
-__device__ __forceinline__ void xg_pin8(float (&v)[8]) {
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]),
-                    "+v"(v[6]), "+v"(v[7]));
-}
-
 template <bool GATE_UP>
 __global__ __launch_bounds__(256, 3) void k_xg_experts(XgExpertArgs a) {
   extern __shared__ __align__(16) char lds[];
@@ -248,9 +241,9 @@ __global__ __launch_bounds__(256, 3) void k_xg_experts(XgExpertArgs a) {
           w[rt][2 * q + 1] = fp4x2_to_f32<2>(cw[q]).x;
         }
         fc[rt] = f[rt];
-        xg_pin8(w[rt]);
+        pin8(w[rt]);
       }
-      xg_pin8(xv);
+      pin8(xv);
       __builtin_amdgcn_sched_barrier(0);
       x0 = x1;
       x1 = x2;

@@ -350,19 +350,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmParams p) {
         *reinterpret_cast<u32x4_t*>(&Ws[buf][((tid + 256 * i) >> 3) * kGS + pc]) = in ? qw[i] : z4;
     }
   };
-  // LDS written before it is read after it; the loads stay on their way
-  auto barrier = [&]() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
 #pragma unroll
   for (int d = 0; d < D; ++d) {
     load_a(d, ra[d]);
     load_w(d, rw[d], rs[d]);
   }
   stage(0, 0, ra[0], rw[0], rs[0]);
-  barrier();
+  lds_barrier();
   // the K loop of a wave with nblk 32-row blocks that hold rows: a block past
   // the tile's rows is not multiplied (nothing of it is stored); of 333 prompt
   // rows an expert of 32 has ~42 of a tile's 128
@@ -395,7 +389,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmParams p) {
         load_w(kt + d + D, rw[d], rs[d]);
         multiply(d & 1);
         stage(kt + d + 1, (d + 1) & 1, ra[(d + 1) % D], rw[(d + 1) % D], rs[(d + 1) % D]);
-        barrier();
+        lds_barrier();
       }
     }
 #pragma unroll
@@ -403,7 +397,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmParams p) {
       if (kt + d < nk) {
         multiply(d & 1);
         stage(kt + d + 1, (d + 1) & 1, ra[d + 1], rw[d + 1], rs[d + 1]);
-        barrier();
+        lds_barrier();
       }
   };
   const int live = (rows - wm * 64 + 31) / 32;  // <= 0: no rows for this wave
