@@ -253,11 +253,13 @@ struct XmStream {
 // serves expert e; a task is 6 intermediate columns (12 rows, gate and up
 // interleaved).  Four of the expert's pairs at a time sit in LDS as fp32, and
 // each wave streams its tasks' rows against them.
-// Bound: the 4x4x1 instruction takes about 9 cycles and the conversions, moves
-// and waits around it as long again (they do not overlap it), so a quad of
-// pairs costs what 1.7 single ones cost the vector kernels; from two pairs per
-// expert on that wins.  20b, B = 16 (64 pairs, 28 experts): gate_up 100 -> 88
-// us, down 57 -> 44 us; B = 64 651 -> 306 us per layer.
+// Bound: matrix instructions and the conversions around them, which do not
+// overlap in a wave (B = 16: matrix units 30% busy, vector units 44%, waves
+// waiting 39% of their time), beside 4.5 TB/s of memory reads, 1.6 times the
+// bytes of the rows: a group's 16 scale bytes fetch a 128-byte line each time.
+// A quad of pairs costs what 1.7 single ones cost the vector kernels; from two
+// pairs per expert on that wins.  20b, B = 16 (64 pairs, 28 experts): gate_up
+// 100 -> 88 us, down 57 -> 44 us; B = 64 616 -> 309 us per layer.
 // ===========================================================================
 constexpr int kXmGuRq = 3;     // row quads per gate_up task
 constexpr int kXmGuTasks = 3;  // tasks per wave

@@ -20,11 +20,13 @@
 // keys (min(S, chunks); the others add nothing to the merge) are numbered in
 // order; each stores its partial and k_xa_merge joins them, or with one of them
 // the block finishes the row.
-// Bound: half of the 16 columns stand empty at G = 8, so the products of a chunk
-// take 2 x 16 x 32 cycles per wave; the exponentials and the barriers come on
-// top.  us, k_attn_split's vector chains -> this with the merge, 64 / 8 heads: B
-// = 8, T = 2048 43.3 -> 21.0, T = 8192 76.6 -> 50.4, B = 32, T = 1024 79 -> 32;
-// 333 prompt rows, 0.79 -> 0.06 ms per layer.
+// Bound: no unit alone.  T = 8192, B = 8: the address units are 54% busy (8-byte
+// loads of K), the vector units 31%, the matrix units 20% (half of the 16 columns
+// stand empty at G = 8), and waves wait 39% of their time, at the two barriers of
+// a chunk among others; memory reads 1.1 times the cache, 2.6 TB/s.
+// us, k_attn_split's vector chains -> this with the merge, 64 / 8 heads: B = 8, T =
+// 2048 44.7 -> 21.6, T = 8192 83.4 -> 51.2, B = 32, T = 1024 79 -> 32; 333 prompt
+// rows, 0.79 -> 0.06 ms per layer.
 #include "neon_common.hpp"
 #include "neon_internal.hpp"
 

@@ -143,8 +143,10 @@ __global__ __launch_bounds__(256) void k_xg_pack_pairs(const uint16_t* __restric
 // The expert products: grid (rows / 32, E), 4 waves.  Block (x, e) holds rows
 // 32 x .. 32 x + 31 of expert e in LDS (codes as stored, scales as bf16), and
 // each wave takes every fourth tile of 16 pairs: two 16 x 16 outputs, the whole
-// K.  The matrix instructions (16 of 32 cycles per unit) set the pace; the
-// inputs of the next four units are on their way.
+// K.  Bound: the chains of a wave, 16 matrix instructions of 32 cycles per unit
+// one after the other, and waves without a tile: the matrix units are 50% busy
+// at 512 rows (4 or 5 tiles per expert; 960 us gate_up, 531 us down) and 40% at
+// 240 rows (626, 354 us).  The inputs of the next three units are on their way.
 //   GATE_UP: SwiGLU of the interleaved (gate, up) rows, which sit in adjacent
 //            registers of a lane, stored as bf16 in the next product's tiles;
 //   DOWN:    ybuf[pair][row] = dot + bias (fp32), combined by k_moe_combine.
