@@ -37,7 +37,8 @@ inline bool moe_wide(int B, int k, int E, int I) {
 // 16 78 / 73, 64 305 / 193; 2048, 1408, 64, 6 B = 16 92 / 102, 21 127 / 120.  The
 // line is for rows that spread.  Rows that all choose the same k experts leave it
 // k x blocks blocks: 2880, k = 4 (160) B = 16 139 / 131, 64 558 / 486, but 2048, k = 4
-// (116) B = 64 242 / 353 and 1024, 2048, 16, 2 (58) B = 64 94 / 158 (spread 111 / 88).
+// (116) B = 64 242 / 353, 1024, 2048, 16, 2 (58) B = 64 94 / 158 (spread 111 / 88)
+// and 160, 512, 32, 3 (24) B = 311 158 / 358 (spread 153 / 121).
 inline bool xm_moe_wanted(int B, int k, int E, int H, int I) {
   const int64_t pairs = B * (int64_t)k;
   const bool many = xm_blocks(I) >= 36;
